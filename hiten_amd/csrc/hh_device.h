@@ -21,8 +21,11 @@
  *           6-double block of the 42-d variational state (b = 0: the state
  *           x, b = 1..6: STM column b-1, b = 7: idle padding).  The state
  *           position is broadcast to the group with DPP moves at every stage,
- *           error norms are reduced across the group with an xor butterfly
- *           (ds_swizzle).
+ *           even lanes form the field's quotients of the first primary, odd
+ *           lanes those of the second, and error norms are reduced across the
+ *           group with an xor butterfly (ds_swizzle).
+ * Both evaluate the field and the error norm without scaled divisions and
+ * special cases (hh_fast.h) where every lane of the wave is in their range.
  */
 #ifndef HH_DEVICE_H
 #define HH_DEVICE_H
@@ -124,6 +127,12 @@ __device__ __forceinline__ double pow_tab(const PowTab* t, double x, double y) {
     return hh_pow_t(x, y, t->invc, t->log_hi, t->log_lo, t->exp_hi, t->exp_lo);
 }
 
+}  // namespace hh
+
+#include "hh_fast.h"
+
+namespace hh {
+
 constexpr int DOP_S = 12;     /* stages of one DOP853 step                 */
 constexpr int DOP_K = 13;     /* stored stage derivatives (k[12] = f(y_high)) */
 constexpr int DOP_SX = 16;    /* stages of the dense-output extension       */
@@ -209,6 +218,48 @@ __device__ __forceinline__ void rhs6(const double (&s)[6], double mu, double (&o
     o[5] = ((-one_mu) * z) / r1c - (mu * z) / r2c;
 }
 
+/* Whether a state and mass take the fast forms (the bounds of FastChk) */
+__device__ __forceinline__ bool rhs6_in_range(const double (&s)[6], double mu) {
+    const double x = s[0], y = s[1], z = s[2];
+    const double xm = x + mu, xr = x - (1.0 - mu);
+    FastChk c;
+    c.dist((xm * xm + y * y) + z * z);
+    c.dist((xr * xr + y * y) + z * z);
+    c.num(xm);
+    c.num((x - 1.0) + mu);
+    c.num(y);
+    c.num(z);
+    c.num(mu);
+    c.num(1.0 - mu);
+    return !c.outside();
+}
+
+/* rhs6 with the fast forms: the three quotients of a primary share one
+ * reciprocal, which starts from the 1/r its square root leaves behind.
+ * 131,072 arcs of Lane6, bound by FP64 issue: 2.37 -> 1.87 ms.            */
+__device__ __forceinline__ void rhs6_fast(const double (&s)[6], double mu, double (&o)[6]) {
+    const double x = s[0], y = s[1], z = s[2], vx = s[3], vy = s[4], vz = s[5];
+    const double xm = x + mu;
+    const double one_mu = 1.0 - mu;
+    const double xr = x - one_mu;
+    const double P1 = (xm * xm + y * y) + z * z;
+    const double P2 = (xr * xr + y * y) + z * z;
+    const double xm1 = (x - 1.0) + mu;
+    double h1, h2;
+    const double r1 = fast_sqrt(P1, h1);
+    const double r2 = fast_sqrt(P2, h2);
+    const double r1c = r1 * (r1 * r1);
+    const double r2c = r2 * (r2 * r2);
+    const double k1 = rcp_step(r1c, (8.0 * h1) * (h1 * h1));
+    const double k2 = rcp_step(r2c, (8.0 * h2) * (h2 * h2));
+    o[0] = vx;
+    o[1] = vy;
+    o[2] = vz;
+    o[3] = ((2.0 * vy + x) - fast_div(one_mu * xm, r1c, k1)) - fast_div(mu * xm1, r2c, k2);
+    o[4] = ((-2.0 * vx + y) - fast_div(one_mu * y, r1c, k1)) - fast_div(mu * y, r2c, k2);
+    o[5] = fast_div((-one_mu) * z, r1c, k1) - fast_div(mu * z, r2c, k2);
+}
+
 /* One STM column p = Phi[:, j] -> (F @ Phi)[:, j] given the Hessian entries
  * of the Jacobian (rtbp.py:124-141).                                       */
 __device__ __forceinline__ void column_rhs(double uxx, double uyy, double uzz, double uxy,
@@ -226,6 +277,14 @@ __device__ __forceinline__ void column_rhs(double uxx, double uyy, double uzz, d
 /* lane layout policies                                                     */
 /* ---------------------------------------------------------------------- */
 
+/* lane q of each aligned quad by DPP: lane i takes lane CTRL[i] */
+template <int CTRL>
+__device__ __forceinline__ double quad_get(double v) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, false);
+    return __hiloint2double(hi, lo);
+}
+
 /* One trajectory per lane, 6-d state. */
 struct Lane6 {
     static constexpr int N = 6;
@@ -234,7 +293,8 @@ struct Lane6 {
     bool flip_on;       /* kernel-uniform: any flip at all                     */
 
     __device__ __forceinline__ void rhs(const double (&s)[6], double (&o)[6]) const {
-        rhs6(s, mu, o);
+        if (__builtin_expect(__any(!rhs6_in_range(s, mu)), 0)) rhs6(s, mu, o);
+        else rhs6_fast(s, mu, o);
         if (flip_on) {
 #pragma unroll
             for (int d = 0; d < 6; ++d) o[d] = neg_if(o[d], flipbits, d);
@@ -259,10 +319,10 @@ struct Lane42 {
     bool flip_on;
     int blk;            /* lane & 7 */
 
-    __device__ __forceinline__ void rhs(const double (&s)[6], double (&o)[6]) const {
-        const double x = bcast8(s[0]);
-        const double y = bcast8(s[1]);
-        const double z = bcast8(s[2]);
+    /* the general form, any argument: every lane forms the six quotients it
+     * needs with IEEE divisions                                           */
+    __device__ __forceinline__ void rhs_general(const double (&s)[6], double x, double y,
+                                                double z, double (&o)[6]) const {
         const bool st = (blk == 0);
         const double xm = x + mu;
         const double xr = x - mu2;
@@ -298,6 +358,76 @@ struct Lane42 {
             const double uxz = (3.0 * z) * gx;
             const double uyz = ((3.0 * y) * z) * (q1 + q2);
             column_rhs(uxx, uyy, uzz, uxy, uxz, uyz, s, o);
+        }
+    }
+
+    /* The fast forms with the two primaries shared out: even lanes form
+     * the powers and quotients of r, odd lanes those of R, three quotients a
+     * lane instead of six -- lanes 0 and 1 the state's (xm/r3, y/r3, z/r3 and
+     * xr/R3, y/R3, z/R3), lanes 2..7 the columns' (mu2/r5, mu2/r3, (mu2
+     * xm)/r5 and mu/R5, mu/R3, (mu xr)/R5) -- and every lane takes the even
+     * and the odd set from its quad with two DPP moves per dword: quad_perm
+     * [0,2,2,2] and [1,3,3,3] give lane 0 its own set and lane 1's, lanes 1..3
+     * the column sets of lanes 2 and 3 (and so in the upper quad, where all
+     * lanes hold column sets).  The kernels of this layout are bound by FP64
+     * issue: with both powers and all six IEEE divisions in every lane the
+     * plain kernel took 354 ms on the 262,144-trajectory uneven batch, with
+     * this form 257 ms, and 10.2 against 7.6 ms on 4,096 trajectories.     */
+    __device__ __forceinline__ void rhs(const double (&s)[6], double (&o)[6]) const {
+        const double x = bcast8(s[0]);
+        const double y = bcast8(s[1]);
+        const double z = bcast8(s[2]);
+        const bool st = (blk == 0);
+        const bool odd = (blk & 1) != 0;
+        const bool sq = (blk < 2);
+        const double xm = x + mu;
+        const double xr = x - mu2;
+        const double xo = odd ? xr : xm;
+        const double m = odd ? mu : mu2;
+        const double y2 = y * y, z2 = z * z;
+        const double P = (xo * xo + y2) + z2;
+        FastChk c;
+        c.dist(P);
+        c.num(xo);
+        c.num(y);
+        c.num(z);
+        c.num(m);
+        if (__builtin_expect(__any(c.outside()), 0)) {
+            rhs_general(s, x, y, z, o);
+        } else {
+            double P3, P5, K3, K5;
+            fast_pow15_25(P, P3, P5, K3, K5);
+            const double D = sq ? P3 : P5, K = sq ? K3 : K5;
+            const double qa = fast_div(sq ? xo : m, D, K);
+            const double qb = fast_div(sq ? y : m, P3, K3);
+            const double qc = fast_div(sq ? z : m * xo, D, K);
+            const double q1 = quad_get<0xA8>(qa), q2 = quad_get<0xFD>(qa);
+            const double q3 = quad_get<0xA8>(qb), q4 = quad_get<0xFD>(qb);
+            const double q5 = quad_get<0xA8>(qc), q6 = quad_get<0xFD>(qc);
+            /* state rows (rtbp.py:233-242) */
+            const double s3 = ((x - mu2 * q1) - mu * q2) + 2.0 * s[4];
+            const double s4 = ((y - mu2 * q3) - mu * q4) - 2.0 * s[3];
+            const double s5 = (-mu2 * q5) - mu * q6;
+            /* Hessian entries (rtbp.py:124-141) and the column rows */
+            const double a53 = q1 * 3.0;
+            const double b53 = q2 * 3.0;
+            const double c3 = q3 + q4;
+            const double gx = q5 + q6;
+            const double uxx = ((1.0 + a53 * (xm * xm)) + b53 * (xr * xr)) - c3;
+            const double uyy = ((1.0 + a53 * y2) + b53 * y2) - c3;
+            const double uzz = ((0.0 + a53 * z2) + b53 * z2) - c3;
+            const double uxy = (3.0 * y) * gx;
+            const double uxz = (3.0 * z) * gx;
+            const double uyz = ((3.0 * y) * z) * (q1 + q2);
+            column_rhs(uxx, uyy, uzz, uxy, uxz, uyz, s, o);
+            /* x + -0.0 is x: the state's rows 0..2 are the velocities as they are */
+            const double zero = st ? -0.0 : 0.0;
+            o[0] = s[3] + zero;
+            o[1] = s[4] + zero;
+            o[2] = s[5] + zero;
+            o[3] = st ? s3 : o[3];
+            o[4] = st ? s4 : o[4];
+            o[5] = st ? s5 : o[5];
         }
         if (flip_on) {
 #pragma unroll
@@ -472,13 +602,34 @@ __device__ __forceinline__ double dop853_attempt(const P& p, const double (&y)[6
         }
     }
     double s5 = 0.0, s3 = 0.0;
+    double sc[6];
+    FastChk c;
 #pragma unroll
     for (int d = 0; d < 6; ++d) {
-        const double sc = atol + rtol * np_max(__builtin_fabs(y[d]), __builtin_fabs(yh[d]));
-        const double q5 = (e5[d] * h) / sc;
-        const double q3 = (e3[d] * h) / sc;
-        s5 += q5 * q5;
-        s3 += q3 * q3;
+        sc[d] = atol + rtol * np_max(__builtin_fabs(y[d]), __builtin_fabs(yh[d]));
+        e5[d] = e5[d] * h;
+        e3[d] = e3[d] * h;
+        c.scale(sc[d]);
+        c.num(e5[d]);
+        c.num(e3[d]);
+    }
+    if (__builtin_expect(__any(c.outside()), 0)) {
+#pragma unroll
+        for (int d = 0; d < 6; ++d) {
+            const double q5 = e5[d] / sc[d];
+            const double q3 = e3[d] / sc[d];
+            s5 += q5 * q5;
+            s3 += q3 * q3;
+        }
+    } else {
+#pragma unroll
+        for (int d = 0; d < 6; ++d) {
+            const double r = fast_rcp(sc[d]);
+            const double q5 = fast_div(e5[d], sc[d], r);
+            const double q3 = fast_div(e3[d], sc[d], r);
+            s5 += q5 * q5;
+            s3 += q3 * q3;
+        }
     }
     s5 = p.reduce(s5);
     s3 = p.reduce(s3);

@@ -1,0 +1,78 @@
+"""GPU: the field and the step loops at the edges of the exponent range in
+which divisions and powers take their unscaled forms (squared distances in
+[2^-100, 2^100), coordinates and masses 0 or at least 2^-301, error scales in
+[2^-300, 2^300)), against the oracle bit for bit: states inside, on either
+side of each bound, and both in one wave."""
+
+import numpy as np
+import pytest
+
+from hiten_amd import batch, workloads as W
+
+pytestmark = pytest.mark.gpu
+
+MU = W.MU_EM
+#: magnitudes on both sides of the bounds 2^-301, 2^-50 (distance), 2^50
+SIZES = [0.0, -0.0, 5e-324, 1e-300, 2.0 ** -302, 2.0 ** -301, 2.0 ** -300, 1e-60, 2.0 ** -51,
+         2.0 ** -50, 2.0 ** -49, 1e-9, 1e-3, 2.0 ** 49, 2.0 ** 50, 2.0 ** 51]
+
+
+def _states():
+    rng = np.random.default_rng(5)
+    rows = []
+    for mu in (MU, 0.0, 2.0 ** -302, 2.0 ** -300, 3.0035e-6):
+        for k, s in enumerate(SIZES):
+            t = SIZES[(k + 5) % len(SIZES)]
+            near = rng.uniform(0.8, 0.9)
+            v = rng.normal(size=3)
+            rows += [(mu, [near, 0.01, s, *v]), (mu, [near, s, t, *v]),
+                     (mu, [-mu + s, 0.0, 0.0, *v]), (mu, [1.0 - mu + s, 0.0, t, *v]),
+                     (mu, [1.0 - mu, s, 0.0, *v]), (mu, [s, s, s, *v])]
+    mus = np.array([r[0] for r in rows])
+    y = np.array([r[1] for r in rows])
+    # a collision (distance 0) has no finite derivative
+    d = np.minimum(np.hypot(np.hypot(y[:, 0] + mus, y[:, 1]), y[:, 2]),
+                   np.hypot(np.hypot(y[:, 0] - (1.0 - mus), y[:, 1]), y[:, 2]))
+    return mus[d > 0], y[d > 0]
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("dim", [6, 42])
+def test_field_at_the_range_bounds(gpu, oracle, dim, mixed):
+    mu, x = _states()
+    rng = np.random.default_rng(6)
+    if mixed:
+        # one edge state among states near L1 in every wave
+        keep = np.arange(len(x)) % (8 if dim == 42 else 64) == 3
+        x[~keep] = W.planar_seeds(rng, int((~keep).sum()))
+        mu[~keep] = MU
+    y = x if dim == 6 else np.concatenate([rng.normal(size=(len(x), 36)), x], axis=1)
+    got = batch.eval_rhs(mu, y, dim=dim).cpu().numpy()
+    f = oracle.crtbp_accel if dim == 6 else oracle.var_equations
+    want = np.array([f(s, m) for s, m in zip(y, mu)])
+    assert np.array_equal(got, want, equal_nan=True)
+
+
+@pytest.mark.parametrize("dim,variant", [(6, "plain"), (6, "wide"), (42, "plain"), (42, "wide"),
+                                         (42, "pair"), (42, "persistent")])
+@pytest.mark.parametrize("n", [1, 9, 130])
+def test_integration_at_the_range_bounds(gpu, oracle, dim, variant, n):
+    """Arcs with out-of-plane motion from 0 to below the bounds, masses on both
+    sides of theirs, one error scale below its bound."""
+    rng = np.random.default_rng(n)
+    x = W.planar_seeds(rng, n)
+    tiny = np.array([0.0, 1e-300, 2.0 ** -302, 2.0 ** -300, 1e-30, 1.0])
+    x[:, 2] *= tiny[np.arange(n) % 6]
+    x[:, 5] = tiny[(np.arange(n) + 2) % 6] * 1e-2
+    mu = np.array([MU, 0.0, 2.0 ** -302, 1e-80])[np.arange(n) % 4]
+    y0 = x if dim == 6 else W.with_identity_stm(x)
+    tf = rng.uniform(0.3, 0.9, n)
+    for atol in (1e-12, 2.0 ** -310):
+        r = batch.dop853_final(mu, y0, 0.0, tf, dim=dim, atol=atol, variant=variant,
+                               max_steps=400)
+        want, na, nr, st = oracle.batch_dop853_final(mu, y0, np.zeros(n), tf, atol=atol,
+                                                     max_steps=400)
+        assert np.array_equal(r.y.cpu().numpy(), want, equal_nan=True)
+        assert np.array_equal(r.n_accepted.cpu().numpy(), na)
+        assert np.array_equal(r.n_rejected.cpu().numpy(), nr)
+        assert np.array_equal(r.status.cpu().numpy(), st)
