@@ -453,19 +453,21 @@ __global__ __launch_bounds__(256) void k_rk_fixed_event6(
     }
 }
 
-/* k_rk_fixed6 with one trajectory per aligned 8-lane group, one component
- * per lane (Group6): rk_run's grid, steps and stores, per component.        */
-template <class M, int BLOCK>
-__global__ __launch_bounds__(BLOCK) void k_rk_fixed6_group(
+/* k_rk_fixed6 with one trajectory per lane group, one component per lane
+ * (P = Group6 or Row6): rk_run's grid, steps and stores, per component.     */
+template <class M, class P>
+__global__ __launch_bounds__(256) void k_rk_fixed6_group(
     int n, const double* __restrict__ mu, const double* __restrict__ t0a,
     const double* __restrict__ tfa, int steps, const double* __restrict__ t_vals, int fwd,
     unsigned long long flip, const double* __restrict__ y0, double* __restrict__ yout,
     double* __restrict__ traj, double* __restrict__ deriv) {
-    const long long gtid = (long long)blockIdx.x * BLOCK + threadIdx.x;
-    const int i = (int)(gtid >> 3);
+    const long long gtid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = (int)(gtid / P::LANES);
     if (i >= n) return;
-    Group6 p;
+    P p;
     p.setup(threadIdx.x & 63, mu[i], fwd, flip, nullptr);   /* no step control */
+    RkRow<M> tab;
+    if constexpr (P::LANES == 16) tab.fill(p.lane);
     const int d = p.d;
     double y = p.act ? y0[(size_t)d * n + i] : 0.0;
     const double t0 = t0a[i], tf = tfa[i];
@@ -479,7 +481,7 @@ __global__ __launch_bounds__(BLOCK) void k_rk_fixed6_group(
         const double t_s = grid_time(t_vals, s_idx, steps, t0, tf, step, delta, zstep);
         if (!constant) {
             double k0;
-            rk_step_group<M>(p, y, t_s - t_prev, k0);
+            rk_step_group<M>(p, tab, y, t_s - t_prev, k0);
             if (deriv && p.act) deriv[((size_t)(s_idx - 1) * 6 + d) * n + i] = k0;
         }
         t_prev = t_s;
@@ -542,9 +544,6 @@ __global__ __launch_bounds__(256) void k_dop853_run6(
     if (nrej) nrej[i] = s.nrej;
 }
 
-/* k_dop853_run6 with one trajectory per aligned 8-lane group, one component
- * per lane (Group6).  traj_init / traj_iterate and the FinalOut / GridOut
- * policies, statement for statement, with each lane holding its component. */
 /* A caller's request to stop a loop early: with CANCEL set, the loops below
  * read the flag (LDS) before each attempt and stop with ST_CANCELLED once it
  * is nonzero.  Without it they compile as before.                         */
@@ -555,12 +554,13 @@ __device__ __forceinline__ bool cancelled(const int* flag) {
     return false;
 }
 
-/* One trajectory of k_dop853_run6 in the Group6 layout, statement for
- * statement: the grid form writes this lane's component of every output
+/* One trajectory of k_dop853_run6 in a lane group (Group6 or Row6):
+ * traj_init / traj_iterate and the FinalOut / GridOut policies, statement for
+ * statement, with each lane holding its component: the grid form writes this lane's component of every output
  * point to gout ([m][6]); the final form returns it in yfin.  Status and
  * counters are the same in all lanes of the group.                         */
-template <bool GRID, bool CANCEL = false>
-__device__ __forceinline__ void group6_run(const Group6& p, double y, double t0, double tf,
+template <bool GRID, bool CANCEL = false, class P>
+__device__ __forceinline__ void group6_run(const P& p, double y, double t0, double tf,
                                            const StepParams& sp, double* gout, int m,
                                            const double* teval, double& yfin, int& status,
                                            int& nacc, int& nrej, const int* cancel = nullptr) {
@@ -664,8 +664,9 @@ __device__ __forceinline__ void group6_run(const Group6& p, double y, double t0,
     nrej = nr;
 }
 
-template <int BLOCK, bool GRID>
-__global__ __launch_bounds__(BLOCK) void k_dop853_run6_group(
+template <class P, bool GRID>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+void k_dop853_run6_group(
     int n, const double* __restrict__ mu, const double* __restrict__ t0a,
     const double* __restrict__ tfa, StepParams sp, int fwd, unsigned long long flip,
     const double* __restrict__ y0, double* __restrict__ yout, int m,
@@ -674,11 +675,12 @@ __global__ __launch_bounds__(BLOCK) void k_dop853_run6_group(
     __shared__ PowTab powt;
     pow_tab_fill(&powt);
     __syncthreads();
-    const long long gtid = (long long)blockIdx.x * BLOCK + threadIdx.x;
-    const int i = (int)(gtid >> 3);
+    const long long gtid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = (int)(gtid / P::LANES);
     if (i >= n) return;
-    Group6 p;
+    P p;
     p.setup(threadIdx.x & 63, mu[i], fwd, flip, &powt);
+    p.dop_setup();
     const int d = p.d;
     const double y = p.act ? y0[(size_t)d * n + i] : 0.0;
     double yfin;
@@ -797,7 +799,10 @@ __global__ __launch_bounds__(256) void k_dop853_event6(
     if (nrej) nrej[i] = nr;
 }
 
-/* One event search of k_dop853_event6 in the Group6 layout, statement for
+/* The lane-group kernels below are held to 128 VGPRs: 32,768 event searches
+ * (8 lanes each) are then resident at once, four waves on every SIMD.       */
+
+/* One event search of k_dop853_event6 in a lane group, statement for
  * statement; the event component is read from its lane of the group.  Per
  * lane: this lane's components of y_hit and y_last; the flags, t_hit and
  * counters are the same in all lanes of the group.                         */
@@ -806,15 +811,15 @@ struct EventOut6 {
     double t_hit, y_hit, y_last;
 };
 
-template <bool CANCEL = false>
-__device__ __forceinline__ void group6_event(const Group6& p, double y, double t, double tmax,
+template <bool CANCEL = false, class P>
+__device__ __forceinline__ void group6_event(const P& p, double y, double t, double tmax,
                                              const StepParams& sp, const EventParams& ev,
                                              EventOut6& o, const int* cancel = nullptr) {
     double k[DOP_K];
 #pragma unroll
     for (int j = 0; j < DOP_K; ++j) k[j] = 0.0;
     k[0] = p.rhs(y);
-    const int ev_addr = p.base + (ev.index << 2);
+    const int ev_addr = p.comp_addr(ev.index);
     double gp = bperm(y, ev_addr) - ev.offset;
     double h = p.initial_step(y, k[0], sp.rtol, sp.atol, sp.min_step, sp.max_step);
     double err_prev = -1.0;
@@ -881,10 +886,11 @@ __device__ __forceinline__ void group6_event(const Group6& p, double y, double t
     o.y_last = ylast;
 }
 
-/* k_dop853_event6 with one trajectory per aligned 8-lane group, one
- * component per lane (Group6): the latency form for small batches.          */
-template <int BLOCK>
-__global__ __launch_bounds__(BLOCK) void k_dop853_event6_group(
+/* k_dop853_event6 with one trajectory per lane group, one component per
+ * lane: the latency form for small batches.                                 */
+template <class P>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+void k_dop853_event6_group(
     int n, const double* __restrict__ mu, const double* __restrict__ t0a,
     const double* __restrict__ tmaxa, StepParams sp, EventParams ev, int fwd,
     unsigned long long flip, const double* __restrict__ y0, int* __restrict__ hit,
@@ -893,11 +899,12 @@ __global__ __launch_bounds__(BLOCK) void k_dop853_event6_group(
     __shared__ PowTab powt;
     pow_tab_fill(&powt);
     __syncthreads();
-    const long long gtid = (long long)blockIdx.x * BLOCK + threadIdx.x;
-    const int i = (int)(gtid >> 3);
+    const long long gtid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = (int)(gtid / P::LANES);
     if (i >= n) return;
-    Group6 p;
+    P p;
     p.setup(threadIdx.x & 63, mu[i], fwd, flip, &powt);
+    p.dop_setup();
     const int d = p.d;
     const double y = p.act ? y0[(size_t)d * n + i] : 0.0;
     EventOut6 o;
@@ -1847,6 +1854,14 @@ StepParams make_sp(double rtol, double atol, double max_step, double min_step,
 /* the device-resident corrector, on the loops above */
 #include "hh_correct.h"
 
+/* Up to this many 6-d trajectories take 16-lane groups (Row6, a shorter
+ * instruction stream), more 8-lane groups (Group6, half the waves).  4,096
+ * trajectories are 1,024 waves of 16-lane groups, one for each SIMD; from
+ * there on waves share SIMDs.  Event searches, 16 against 8 lanes: 0.39 and
+ * 0.40 ms at 8,192, 0.61 and 0.56 ms at 16,384, 0.89 and 0.59 ms at 32,768;
+ * end states 0.64 and 0.62 ms at 8,192, 1.78 and 1.42 ms at 65,536.         */
+constexpr int ROW6_MAX = 4096;
+
 template <class M>
 void launch_rk_fixed(int n, int dim, const double* mu, const double* t0p,
                             const double* tfp, int steps, const double* t_vals, int fwd,
@@ -1854,13 +1869,16 @@ void launch_rk_fixed(int n, int dim, const double* mu, const double* t0p,
                             double* traj_out, double* deriv_out, int variant, int block,
                             hipStream_t st) {
     if (dim == 6 && variant == HH_VARIANT_WIDE) {
-        const int g = blocks_for((long long)n * 8, block);
-        switch (block) {
-            case 64: hipLaunchKernelGGL((k_rk_fixed6_group<M, 64>), dim3(g), dim3(64), 0, st, n, mu, t0p, tfp, steps, t_vals, fwd, flip_mask, y0, y_out, traj_out, deriv_out); break;
-            case 128: hipLaunchKernelGGL((k_rk_fixed6_group<M, 128>), dim3(g), dim3(128), 0, st, n, mu, t0p, tfp, steps, t_vals, fwd, flip_mask, y0, y_out, traj_out, deriv_out); break;
-            case 192: hipLaunchKernelGGL((k_rk_fixed6_group<M, 192>), dim3(g), dim3(192), 0, st, n, mu, t0p, tfp, steps, t_vals, fwd, flip_mask, y0, y_out, traj_out, deriv_out); break;
-            default: hipLaunchKernelGGL((k_rk_fixed6_group<M, 256>), dim3(g), dim3(256), 0, st, n, mu, t0p, tfp, steps, t_vals, fwd, flip_mask, y0, y_out, traj_out, deriv_out); break;
-        }
+        if (n <= ROW6_MAX)
+            hipLaunchKernelGGL((k_rk_fixed6_group<M, Row6>),
+                               dim3(blocks_for((long long)n * 16, block)), dim3(block), 0, st, n,
+                               mu, t0p, tfp, steps, t_vals, fwd, flip_mask, y0, y_out, traj_out,
+                               deriv_out);
+        else
+            hipLaunchKernelGGL((k_rk_fixed6_group<M, Group6>),
+                               dim3(blocks_for((long long)n * 8, block)), dim3(block), 0, st, n,
+                               mu, t0p, tfp, steps, t_vals, fwd, flip_mask, y0, y_out, traj_out,
+                               deriv_out);
     } else if (dim == 6) {
         hipLaunchKernelGGL(k_rk_fixed6<M>, dim3(blocks_for(n, block)), dim3(block), 0, st, n, mu,
                            t0p, tfp, steps, t_vals, fwd, flip_mask, y0, y_out, traj_out,
@@ -1882,13 +1900,14 @@ static int launch_run6_group(int n, const double* mu, const double* t0, const do
                              StepParams sp, int fwd, unsigned long long flip, const double* y0,
                              double* out, int m, const double* teval, int* status, int* nacc,
                              int* nrej, int block, hipStream_t st, const char* what) {
-    const int g = blocks_for((long long)n * 8, block);
-    switch (block) {
-        case 64: hipLaunchKernelGGL((k_dop853_run6_group<64, GRID>), dim3(g), dim3(64), 0, st, n, mu, t0, tf, sp, fwd, flip, y0, out, m, teval, status, nacc, nrej); break;
-        case 128: hipLaunchKernelGGL((k_dop853_run6_group<128, GRID>), dim3(g), dim3(128), 0, st, n, mu, t0, tf, sp, fwd, flip, y0, out, m, teval, status, nacc, nrej); break;
-        case 192: hipLaunchKernelGGL((k_dop853_run6_group<192, GRID>), dim3(g), dim3(192), 0, st, n, mu, t0, tf, sp, fwd, flip, y0, out, m, teval, status, nacc, nrej); break;
-        default: hipLaunchKernelGGL((k_dop853_run6_group<256, GRID>), dim3(g), dim3(256), 0, st, n, mu, t0, tf, sp, fwd, flip, y0, out, m, teval, status, nacc, nrej); break;
-    }
+    if (n <= ROW6_MAX)
+        hipLaunchKernelGGL((k_dop853_run6_group<Row6, GRID>),
+                           dim3(blocks_for((long long)n * 16, block)), dim3(block), 0, st, n, mu,
+                           t0, tf, sp, fwd, flip, y0, out, m, teval, status, nacc, nrej);
+    else
+        hipLaunchKernelGGL((k_dop853_run6_group<Group6, GRID>),
+                           dim3(blocks_for((long long)n * 8, block)), dim3(block), 0, st, n, mu,
+                           t0, tf, sp, fwd, flip, y0, out, m, teval, status, nacc, nrej);
     return check_launch(what);
 }
 
@@ -2279,13 +2298,16 @@ int hh_dop853_event(int n, const double* mu, const double* t0, const double* tma
     ev.index = ev_index; ev.offset = ev_offset; ev.direction = direction; ev.xtol = xtol; ev.gtol = gtol;
     hipStream_t st = (hipStream_t)stream;
     if (variant == HH_VARIANT_WIDE) {
-        const int g = blocks_for((long long)n * 8, block);
-        switch (block) {
-            case 64: hipLaunchKernelGGL(k_dop853_event6_group<64>, dim3(g), dim3(64), 0, st, n, mu, t0, tmax, sp, ev, fwd, flip_mask, y0, hit, t_hit, y_hit, y_last, status, n_acc, n_rej); break;
-            case 128: hipLaunchKernelGGL(k_dop853_event6_group<128>, dim3(g), dim3(128), 0, st, n, mu, t0, tmax, sp, ev, fwd, flip_mask, y0, hit, t_hit, y_hit, y_last, status, n_acc, n_rej); break;
-            case 192: hipLaunchKernelGGL(k_dop853_event6_group<192>, dim3(g), dim3(192), 0, st, n, mu, t0, tmax, sp, ev, fwd, flip_mask, y0, hit, t_hit, y_hit, y_last, status, n_acc, n_rej); break;
-            default: hipLaunchKernelGGL(k_dop853_event6_group<256>, dim3(g), dim3(256), 0, st, n, mu, t0, tmax, sp, ev, fwd, flip_mask, y0, hit, t_hit, y_hit, y_last, status, n_acc, n_rej); break;
-        }
+        if (n <= ROW6_MAX)
+            hipLaunchKernelGGL(k_dop853_event6_group<Row6>,
+                               dim3(blocks_for((long long)n * 16, block)), dim3(block), 0, st, n,
+                               mu, t0, tmax, sp, ev, fwd, flip_mask, y0, hit, t_hit, y_hit,
+                               y_last, status, n_acc, n_rej);
+        else
+            hipLaunchKernelGGL(k_dop853_event6_group<Group6>,
+                               dim3(blocks_for((long long)n * 8, block)), dim3(block), 0, st, n,
+                               mu, t0, tmax, sp, ev, fwd, flip_mask, y0, hit, t_hit, y_hit,
+                               y_last, status, n_acc, n_rej);
         return check_launch("hh_dop853_event (group) launch");
     }
     if (variant != HH_VARIANT_PLAIN) return fail(HH_ERR_ARGS, "hh_dop853_event: variant must be PLAIN or WIDE");

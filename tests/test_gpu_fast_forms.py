@@ -76,3 +76,31 @@ def test_integration_at_the_range_bounds(gpu, oracle, dim, variant, n):
         assert np.array_equal(r.n_accepted.cpu().numpy(), na)
         assert np.array_equal(r.n_rejected.cpu().numpy(), nr)
         assert np.array_equal(r.status.cpu().numpy(), st)
+
+
+@pytest.mark.parametrize("n", [3, 4096, 4097])
+def test_lane_groups_on_either_side_of_their_size_rule(gpu, n):
+    """The 16- and 8-lane groups of the "wide" forms (up to 4,096 trajectories,
+    more) against one trajectory per lane: fixed steps of every order, end
+    states, grids and events, forward and backward, bit for bit."""
+    rng = np.random.default_rng(n)
+    y = W.planar_seeds(rng, n)
+    y[:, 1] = rng.uniform(-0.02, 0.02, n)
+    tf = rng.uniform(0.2, 1.5, n)
+
+    def same(f):
+        a, b = f("wide"), f("plain")
+        for u, v in zip(a, b):
+            assert np.array_equal(u.cpu().numpy(), v.cpu().numpy())
+
+    for fwd in (1, -1):
+        for order in (4, 6, 8):
+            same(lambda v: batch.rk_fixed(MU, y, 0.0, tf, 9, order=order, forward=fwd,
+                                          return_derivatives=True, variant=v))
+        kw = dict(forward=fwd, flip_indices=slice(0, 6) if fwd < 0 else None)
+        same(lambda v: vars(batch.dop853_final(MU, y, 0.0, tf, variant=v, **kw)).values())
+        same(lambda v: vars(batch.dop853_grid(MU, y, 0.0, tf, 7, variant=v, **kw)).values())
+        same(lambda v: vars(batch.dop853_event(MU, y, 0.0, tf, variant=v, ev_index=1,
+                                               **kw)).values())
+        same(lambda v: vars(batch.dop853_event(MU, y, 0.0, tf, variant=v, ev_index=5,
+                                               direction=1, **kw)).values())
