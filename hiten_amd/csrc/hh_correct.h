@@ -277,14 +277,7 @@ __device__ __forceinline__ int corr_spec_stm(const Wave42& W, const StepParams& 
     for (int j = 0; j < DOP_K; ++j) k[j] = 0.0;
     k[0] = W.rhs(y0);
     const double k00 = k[0];
-    const double sc = sp.atol + sp.rtol * __builtin_fabs(y0);
-    const double ua = y0 / sc;
-    const double ub = k[0] / sc;
-    const double s0 = W.block_tree(W.act ? ua * ua : 0.0);
-    const double s1 = W.block_tree(W.act ? ub * ub : 0.0);
-    const double sn = __builtin_sqrt(42.0);
-    const double h0 = select_initial_step(__builtin_sqrt(s0) / sn, __builtin_sqrt(s1) / sn,
-                                          sp.min_step, sp.max_step);
+    const double h0 = W.initial_step(y0, k00, sp);
     /* current state */
     double y = y0, t = 0.0, h = h0, ep = -1.0;
     int na = 0, nr = 0;
@@ -339,8 +332,11 @@ __device__ __forceinline__ int corr_spec_stm(const Wave42& W, const StepParams& 
     } else if (rB >= tf) {
         y = yB; k[0] = kB; t = tB; h = hB; ep = epB; na = naB; nr = nrB;
     }
+    WideFinal o;
     int status;
-    wide_loop(sp, W, y, k, t, tf, h, ep, na, nr, out, status);
+    o.stop(y);
+    wide_loop(sp, W, y, k, t, tf, h, ep, na, nr, o, status);
+    out = o.v;
     nacc_out = na;
     return 1;
 }
@@ -349,32 +345,19 @@ __device__ __forceinline__ int corr_spec_stm(const Wave42& W, const StepParams& 
  * (k_dop853_final42_wide's loop).                                         */
 __device__ __forceinline__ void corr_stm(const Wave42& W, const StepParams& sp, double y0,
                                          double tf, double& out, int& nacc) {
+    WideFinal o;
+    int status, nr;
     nacc = 0;
-    if (isclose(0.0, tf) || !((0.0 - tf) * 1.0 < 0.0)) {
-        out = y0;
-        return;
-    }
-    double k[DOP_K];
-#pragma unroll
-    for (int j = 0; j < DOP_K; ++j) k[j] = 0.0;
-    k[0] = W.rhs(y0);
-    const double sc = sp.atol + sp.rtol * __builtin_fabs(y0);
-    const double ua = y0 / sc;
-    const double ub = k[0] / sc;
-    const double s0 = W.block_tree(W.act ? ua * ua : 0.0);
-    const double s1 = W.block_tree(W.act ? ub * ub : 0.0);
-    const double sn = __builtin_sqrt(42.0);
-    const double h = select_initial_step(__builtin_sqrt(s0) / sn, __builtin_sqrt(s1) / sn,
-                                         sp.min_step, sp.max_step);
-    int nr = 0, status;
-    wide_loop(sp, W, y0, k, 0.0, tf, h, -1.0, nacc, nr, out, status);
+    o.stop(y0);
+    if (!no_span(0.0, tf)) wide_from_start(sp, W, y0, 0.0, tf, o, status, nacc, nr);
+    out = o.v;
 }
 
 /* This lane's component of [I | state]: the identity block of Phi, then
  * the full 6-d state of the controls q.                                   */
 __device__ __forceinline__ double corr_stm_start(const Wave42& W, const hh::NewtonRow& w,
                                                  const double* q) {
-    if (!W.holds()) return 0.0;
+    if (!W.holds()) return W.idle();
     const int c = W.comp();
     if (c < 36) return (c / 6 == c % 6) ? 1.0 : 0.0;
     double v = w.base[c - 36];
@@ -397,6 +380,7 @@ __device__ __forceinline__ double corr_stm_start(const Wave42& W, const hh::Newt
 __global__ __launch_bounds__(192) void k_correct(CorrArgs a) {
     __shared__ CorrLds L;
     __shared__ PowTab powt;
+    __shared__ StageRec rec, zero;
     const int i = blockIdx.x;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -404,6 +388,7 @@ __global__ __launch_bounds__(192) void k_correct(CorrArgs a) {
     const int wid = __builtin_amdgcn_readfirstlane((int)(tid >> 6));
     if (i >= a.n) return;
     pow_tab_fill(&powt);
+    wave_lds_clear(zero);
     if (tid == 0) {
         const hh_correction_t& pb = a.prob[i];
         L.fail = 1;
@@ -430,7 +415,7 @@ __global__ __launch_bounds__(192) void k_correct(CorrArgs a) {
         ga.setup(lane, mu, L.row.fwd, a.x.flip_align, &powt);
         ge.setup(lane, mu, 1, 0ULL, &powt);
         Wave42 W;
-        W.setup(lane, mu, 1, a.flip_stm, &powt);
+        W.setup(lane, mu, 1, a.flip_stm, &powt, &rec, &zero);
         for (;;) {
             /* the residual, or the line-search trials of the step; the STM
              * wave meanwhile integrates state 0's STM                      */

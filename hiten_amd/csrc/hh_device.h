@@ -145,6 +145,12 @@ constexpr int ST_CANCELLED = 3;   /* stopped by its caller; the result is not us
 constexpr int ST_DROPPED = 4;     /* lost by the persistent scheduler (ruled out by its
                                      queue capacity; reported rather than silent)     */
 
+/* tolerances, step bounds and the attempt bound of an integration */
+struct StepParams {
+    double rtol, atol, max_step, min_step;
+    long long max_steps;
+};
+
 __device__ __forceinline__ double np_max(double a, double b) {
     /* numpy.maximum: NaN-propagating */
     if (a != a || b != b) return a + b;

@@ -31,10 +31,13 @@ namespace hh {
 /* Extreme exponents seen by the fast forms.  Squared distances must lie in
  * [2^-100, 2^100), the coordinates they come from (and so the numerators)
  * must be 0 or at least 2^-301 in magnitude, error scales in
- * [2^-300, 2^300).  NaN and infinities fail the first test.               */
+ * [2^-300, 2^960): the scale of an STM entry is rtol times the entry, and the
+ * entries of a trajectory that runs into a primary grow to 1e300 over
+ * thousands of attempts.  A quotient by a scale that falls below the normal
+ * range has the square 0 either way.  NaN and infinities fail the first test. */
 struct FastChk {
     static constexpr unsigned DIST_LO = (1023u - 100u) << 20, DIST_SPAN = 200u << 20;
-    static constexpr unsigned SCALE_LO = (1023u - 300u) << 20, SCALE_SPAN = 600u << 20;
+    static constexpr unsigned SCALE_LO = (1023u - 300u) << 20, SCALE_SPAN = 1260u << 20;
     unsigned dist_max = 0, scale_max = 0;
     int num_min = 0;
 

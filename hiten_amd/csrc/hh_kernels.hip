@@ -68,10 +68,6 @@ __device__ __forceinline__ unsigned lane_flip_bits(int fwd, unsigned long long f
 /* ------------------------------------------------------------------------ */
 /* per-trajectory DOP853 state machine, final-value mode                     */
 /* ------------------------------------------------------------------------ */
-struct StepParams {
-    double rtol, atol, max_step, min_step;
-    long long max_steps;
-};
 
 template <class P>
 struct Traj {
@@ -1023,21 +1019,33 @@ struct NoHook {
     __device__ __forceinline__ void end() {}
 };
 
-/* traj_iterate + FinalOut for one trajectory in a wave-wide layout (Wave42
- * or Pair42), from the current (y, k[0], t, h, err_prev, counters) to its
- * end: this lane's component of the final state in `out`.                  */
-template <class WL, class Hook = NoHook>
+/* Output policy of wide_loop: this lane's component of the final state */
+struct WideFinal {
+    double v;
+    __device__ __forceinline__ void stop(double y) { v = y; }
+    template <class WL>
+    __device__ __forceinline__ void accepted(const WL& W, double y, double yh,
+                                             const double (&k)[DOP_K], double t, double t_new,
+                                             double tf, bool last) {
+        if (!last) return;
+        const double hs = t_new - t;
+        v = (hs == 0.0) ? y : dop853_dense_at(W, y, yh, k, hs, (tf - t) / hs);
+    }
+};
+
+/* traj_iterate for one trajectory in a wave-wide layout (Wave42 or Pair42),
+ * from the current (y, k[0], t, h, err_prev, counters) to its end          */
+template <class WL, class Out, class Hook = NoHook>
 __device__ __forceinline__ void wide_loop(const StepParams& sp, const WL& W, double y,
                                           double (&k)[DOP_K], double t, double tf, double h,
-                                          double err_prev, int& nacc, int& nrej, double& out,
+                                          double err_prev, int& nacc, int& nrej, Out& o,
                                           int& status, Hook hook = Hook()) {
-    out = y;
     status = ST_OK;
     for (;;) {
         hook.attempt(nacc + nrej, t);
         if (nacc + nrej >= sp.max_steps) {
             status = ST_MAXSTEPS;
-            out = y;
+            o.stop(y);
             break;
         }
         double hh = clamp_step(h, sp.max_step, sp.min_step);
@@ -1046,7 +1054,7 @@ __device__ __forceinline__ void wide_loop(const StepParams& sp, const WL& W, dou
         const double err = W.attempt(y, k, hh, sp.rtol, sp.atol, yh);
         if (err != err) {
             status = ST_NONFINITE;
-            out = y;
+            o.stop(y);
             break;
         }
         double fa, fr;
@@ -1054,10 +1062,7 @@ __device__ __forceinline__ void wide_loop(const StepParams& sp, const WL& W, dou
         if (err <= 1.0) {
             const double t_new = t + hh;
             const bool last = !((t_new - tf) * 1.0 < 0.0);
-            if (last) {
-                const double hs = t_new - t;
-                out = (hs == 0.0) ? y : W.dense_at(y, yh, k, hs, (tf - t) / hs);
-            }
+            o.accepted(W, y, yh, k, t, t_new, tf, last);
             t = t_new;
             y = yh;
             k[0] = k[DOP_S];
@@ -1073,15 +1078,31 @@ __device__ __forceinline__ void wide_loop(const StepParams& sp, const WL& W, dou
     hook.end();
 }
 
-/* wide_loop, then the stores of store42 */
-template <class WL, class Hook = NoHook>
-__device__ __forceinline__ void wide_finish(const Final42Args& a, const WL& W, int traj,
-                                            double y, double (&k)[DOP_K], double t, double tf,
-                                            double h, double err_prev, int nacc, int nrej,
-                                            Hook hook = Hook()) {
-    double out;
-    int status;
-    wide_loop(a.sp, W, y, k, t, tf, h, err_prev, nacc, nrej, out, status, hook);
+/* wide_loop from the start: traj_init (rk.py:2441-2448) with the block-tree
+ * sums of Lane42.  The span is neither zero nor reversed.                  */
+template <class WL, class Out>
+__device__ __forceinline__ void wide_from_start(const StepParams& sp, const WL& W, double y0,
+                                                double t0, double tf, Out& o, int& status,
+                                                int& nacc, int& nrej) {
+    nacc = 0;
+    nrej = 0;
+    double k[DOP_K];
+#pragma unroll
+    for (int j = 0; j < DOP_K; ++j) k[j] = 0.0;
+    k[0] = W.template rhs<0>(y0);
+    const double h = W.initial_step(y0, k[0], sp);
+    wide_loop(sp, W, y0, k, t0, tf, h, -1.0, nacc, nrej, o, status);
+}
+
+/* a span that leaves y0 unchanged: zero or reversed (dynamics/base.py:421-424) */
+__device__ __forceinline__ bool no_span(double t0, double tf) {
+    return isclose(t0, tf) || !((t0 - tf) * 1.0 < 0.0);
+}
+
+/* the stores of store42 */
+template <class WL>
+__device__ __forceinline__ void wide_store(const Final42Args& a, const WL& W, int traj, double out,
+                                           int status, int nacc, int nrej) {
     if (W.holds()) a.yout[(size_t)W.comp() * a.n + traj] = out;
     if (W.leader()) {
         if (a.status) a.status[traj] = status;
@@ -1090,18 +1111,32 @@ __device__ __forceinline__ void wide_finish(const Final42Args& a, const WL& W, i
     }
 }
 
+/* wide_loop, then the stores of store42 */
+template <class WL, class Hook = NoHook>
+__device__ __forceinline__ void wide_finish(const Final42Args& a, const WL& W, int traj,
+                                            double y, double (&k)[DOP_K], double t, double tf,
+                                            double h, double err_prev, int nacc, int nrej,
+                                            Hook hook = Hook()) {
+    WideFinal o;
+    int status;
+    o.stop(y);
+    wide_loop(a.sp, W, y, k, t, tf, h, err_prev, nacc, nrej, o, status, hook);
+    wide_store(a, W, traj, o.v, status, nacc, nrej);
+}
+
 /* Finish the trajectory of the group whose lane 0 is `src` with the
- * wave-wide layout: lane 8*b + d takes entry d of block b from lane src + b.
+ * wave-wide layout: the lane of entry d of block b takes it from lane src + b.
  * Raises the wave's issue priority meanwhile: such a trajectory is the
  * longest-running work on its SIMD.                                         */
 template <class Hook = NoHook>
-__device__ __forceinline__ void run_wide(const Final42Args& a, const PowTab* pt, int lane, int src,
+__device__ __forceinline__ void run_wide(const Final42Args& a, const PowTab* pt, StageRec* rec,
+                                         const StageRec* zero, int lane, int src,
                                          int traj_lane, const Lane42& p, const Traj<Lane42>& s,
                                          Hook hook = Hook()) {
     Wave42 W;
-    W.setup(lane, rlane(p.mu, src), a.fwd, a.flip, pt);
-    const int from = src + (lane >> 3);
-    double y = 0.0;
+    W.setup(lane, rlane(p.mu, src), a.fwd, a.flip, pt, rec, zero);
+    const int from = src + W.block();
+    double y = W.idle();
     double k[DOP_K];
 #pragma unroll
     for (int j = 0; j < DOP_K; ++j) k[j] = 0.0;
@@ -1122,102 +1157,70 @@ __device__ __forceinline__ void run_wide(const Final42Args& a, const PowTab* pt,
     __builtin_amdgcn_s_setprio(0);
 }
 
-/* One trajectory per wave from the start (latency form for small batches):
- * traj_init (rk.py:2441-2448) in the wave-wide layout, then wide_finish.    */
+/* One trajectory per wave from the start (latency form for small batches) */
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_dop853_final42_wide(Final42Args a) {
     __shared__ PowTab powt;
+    __shared__ StageRec rec[BLOCK / 64], zero;
     pow_tab_fill(&powt);
+    wave_lds_clear(zero);
     __syncthreads();
     const int traj = (int)((blockIdx.x * (unsigned)BLOCK + threadIdx.x) >> 6);
     const int lane = threadIdx.x & 63;
     if (traj >= a.n) return;
     Wave42 W;
-    W.setup(lane, a.mu[traj], a.fwd, a.flip, &powt);
-    const double y0 = W.act ? a.y0[(size_t)comp42(lane >> 3, W.d) * a.n + traj] : 0.0;
+    W.setup(lane, a.mu[traj], a.fwd, a.flip, &powt, &rec[threadIdx.x >> 6], &zero);
+    const double y0 = W.act ? a.y0[(size_t)W.comp() * a.n + traj] : W.idle();
     const double t0 = a.t0[traj], tf = a.tf[traj];
-    if (isclose(t0, tf) || !((t0 - tf) * 1.0 < 0.0)) {
-        /* zero or reversed span: y0 unchanged (dynamics/base.py:421-424) */
-        if (W.act) a.yout[(size_t)comp42(lane >> 3, W.d) * a.n + traj] = y0;
-        if (lane == 0) {
-            if (a.status) a.status[traj] = ST_OK;
-            if (a.nacc) a.nacc[traj] = 0;
-            if (a.nrej) a.nrej[traj] = 0;
-        }
-        return;
-    }
-    double k[DOP_K];
-#pragma unroll
-    for (int j = 0; j < DOP_K; ++j) k[j] = 0.0;
-    k[0] = W.rhs(y0);
-    /* initial_step with the block-tree sums of Lane42 */
-    const StepParams& sp = a.sp;
-    const double sc = sp.atol + sp.rtol * __builtin_fabs(y0);
-    const double ua = y0 / sc;
-    const double ub = k[0] / sc;
-    const double s0 = W.block_tree(W.act ? ua * ua : 0.0);
-    const double s1 = W.block_tree(W.act ? ub * ub : 0.0);
-    const double sn = __builtin_sqrt(42.0);
-    const double d0 = __builtin_sqrt(s0) / sn;
-    const double d1 = __builtin_sqrt(s1) / sn;
-    const double h = select_initial_step(d0, d1, sp.min_step, sp.max_step);
-    wide_finish(a, W, traj, y0, k, t0, tf, h, -1.0, 0, 0);
+    WideFinal o;
+    int status = ST_OK, nacc = 0, nrej = 0;
+    o.stop(y0);
+    if (!no_span(t0, tf)) wide_from_start(a.sp, W, y0, t0, tf, o, status, nacc, nrej);
+    wide_store(a, W, traj, o.v, status, nacc, nrej);
 }
 
 /* One trajectory per pair of waves (128-thread workgroup) from the start:
- * the state wave and the STM wave of Pair42 side by side on two SIMDs.
- * traj_init (rk.py:2441-2448) with the block-tree sums of Lane42, then
- * wide_loop; a zero or reversed span leaves y0 unchanged
- * (dynamics/base.py:421-424).  Both waves of the workgroup must call it.   */
-__device__ __forceinline__ void pair_final(const Pair42& P, const StepParams& sp, double y0,
-                                           double t0, double tf, double& out, int& status,
-                                           int& nacc, int& nrej) {
-    nacc = 0;
-    nrej = 0;
-    if (isclose(t0, tf) || !((t0 - tf) * 1.0 < 0.0)) {
-        out = y0;
-        status = ST_OK;
-        return;
-    }
-    double k[DOP_K];
-#pragma unroll
-    for (int j = 0; j < DOP_K; ++j) k[j] = 0.0;
-    k[0] = P.rhs(y0);
-    const double sc = sp.atol + sp.rtol * __builtin_fabs(y0);
-    const double ua = y0 / sc;
-    const double ub = k[0] / sc;
-    double s0, s1;
-    P.pair_tree(P.holds() ? ua * ua : 0.0, P.holds() ? ub * ub : 0.0, s0, s1);
-    const double sn = __builtin_sqrt(42.0);
-    const double d0 = __builtin_sqrt(s0) / sn;
-    const double d1 = __builtin_sqrt(s1) / sn;
-    const double h = select_initial_step(d0, d1, sp.min_step, sp.max_step);
-    wide_loop(sp, P, y0, k, t0, tf, h, -1.0, nacc, nrej, out, status);
+ * the state wave and the STM wave of Pair42 side by side on two SIMDs.  Both
+ * waves take the same branches and so meet the same barriers.               */
+template <int ROLE>
+__device__ __forceinline__ void pair_from_start(const Final42Args& a, PairLds* lds,
+                                                const PowTab* pt, int traj, int lane) {
+    Pair42<ROLE> P;
+    P.setup(lane, a.mu[traj], a.fwd, a.flip, lds, pt);
+    const double y0 = P.holds() ? a.y0[(size_t)P.comp() * a.n + traj] : P.idle();
+    const double t0 = a.t0[traj], tf = a.tf[traj];
+    WideFinal o;
+    int status = ST_OK, nacc = 0, nrej = 0;
+    o.stop(y0);
+    if (!no_span(t0, tf)) wide_from_start(a.sp, P, y0, t0, tf, o, status, nacc, nrej);
+    wide_store(a, P, traj, o.v, status, nacc, nrej);
 }
 
 __global__ __launch_bounds__(128) void k_dop853_final42_pair(Final42Args a) {
     __shared__ PairLds lds;
     __shared__ PowTab powt;
     pow_tab_fill(&powt);
+    pair_lds_clear(lds);
     __syncthreads();
     const int traj = blockIdx.x;
     const int lane = threadIdx.x & 63;
-    /* wave-uniform in a scalar register, so that every branch on the role is
-     * a uniform one and each wave executes exactly its own barriers */
-    const int role = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     if (traj >= a.n) return;
-    Pair42 P;
-    P.setup(lane, role, a.mu[traj], a.fwd, a.flip, &lds, &powt);
-    const double y0 = P.holds() ? a.y0[(size_t)P.comp() * a.n + traj] : 0.0;
-    double out;
-    int status, nacc, nrej;
-    pair_final(P, a.sp, y0, a.t0[traj], a.tf[traj], out, status, nacc, nrej);
-    if (P.holds()) a.yout[(size_t)P.comp() * a.n + traj] = out;
-    if (P.leader()) {
-        if (a.status) a.status[traj] = status;
-        if (a.nacc) a.nacc[traj] = nacc;
-        if (a.nrej) a.nrej[traj] = nrej;
-    }
+    /* the role in a scalar register: the branch is a uniform one */
+    if (__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) == 0)
+        pair_from_start<0>(a, &lds, &powt, traj, lane);
+    else
+        pair_from_start<1>(a, &lds, &powt, traj, lane);
+}
+
+/* A wave that has handed its trajectories on forgets them: their registers are
+ * not kept across the wave-wide or pair run that follows                   */
+__device__ __forceinline__ void forget42(Lane42& p, Traj<Lane42>& s, FinalOut& o) {
+    p.mu = p.mu2 = 0.0;
+#pragma unroll
+    for (int d = 0; d < 6; ++d) s.y[d] = s.k[0][d] = o.y[d] = 0.0;
+    s.t = s.tf = s.h = s.err_prev = 0.0;
+    s.nacc = s.nrej = s.status = 0;
+    s.done = true;
 }
 
 /* Work-stealing form.  Each wave keeps its 8 groups busy: after every step
@@ -1230,7 +1233,9 @@ template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void k_dop853_final42_persist(Final42Args a) {
     __shared__ PowTab powt;
+    __shared__ StageRec rec[BLOCK / 64], zero;
     pow_tab_fill(&powt);
+    wave_lds_clear(zero);
     __syncthreads();
     const int lane = threadIdx.x & 63;
     const int b = lane & 7;
@@ -1288,7 +1293,9 @@ void k_dop853_final42_persist(Final42Args a) {
         const unsigned long long live = __ballot(traj >= 0 && b == 0);
         if (__popcll(live) == 1 && (hold || __any(exhausted))) {
             /* one trajectory left in the wave: finish it one component per lane */
-            run_wide(a, &powt, lane, __ffsll((long long)live) - 1, traj, p, s);
+            run_wide(a, &powt, &rec[threadIdx.x >> 6], &zero, lane,
+                     __ffsll((long long)live) - 1, traj, p, s);
+            forget42(p, s, o);
             traj = -1;
             continue;
         }
@@ -1460,14 +1467,16 @@ __device__ __forceinline__ void resume42(const Final42Args& a, const ResumeArgs&
     s.done = false;
 }
 
-/* Finish the handed-over trajectory with both waves of the workgroup */
+/* Finish the handed-over trajectory with both waves of the workgroup, this
+ * one in the given role                                                     */
+template <int ROLE>
 __device__ __forceinline__ void run_pair(const Final42Args& a, const ResumeArgs& r,
                                          const PairHandoff& ho, PairLds* plds, const PowTab* pt,
-                                         int wid, int lane, int key) {
-    Pair42 P;
-    P.setup(lane, wid, ho.mu, a.fwd, a.flip, plds, pt);
-    const int bb = lane >> 3, dd = lane & 7;
-    const double y = P.holds() ? ho.y[bb][dd] : 0.0;
+                                         int lane, int key) {
+    Pair42<ROLE> P;
+    P.setup(lane, ho.mu, a.fwd, a.flip, plds, pt);
+    const int bb = P.block(), dd = P.d;
+    const double y = P.holds() ? ho.y[bb][dd] : P.idle();
     double k[DOP_K];
 #pragma unroll
     for (int j = 0; j < DOP_K; ++j) k[j] = 0.0;
@@ -1500,6 +1509,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE, WPE)
 void k_dop853_final42_resume(Final42Args a, ResumeArgs r) {
     static_assert(BLOCK == 128, "the pair form takes two waves per workgroup");
     __shared__ PairLds plds;
+    __shared__ StageRec rec[2];
     __shared__ PairHandoff ho;
     __shared__ int pair_state;
     __shared__ PowTab powt;
@@ -1509,6 +1519,7 @@ void k_dop853_final42_resume(Final42Args a, ResumeArgs r) {
     const int grp = lane >> 3;
     if (threadIdx.x == 0) pair_state = -1;
     pow_tab_fill(&powt);
+    pair_lds_clear(plds);
     __syncthreads();
     const int key = simd_key();
     Lane42 p;
@@ -1577,7 +1588,9 @@ void k_dop853_final42_resume(Final42Args a, ResumeArgs r) {
             }
             traj = -1;
             __syncthreads();
-            run_pair(a, r, ho, &plds, &powt, wid, lane, key);
+            if (wid == 0) run_pair<0>(a, r, ho, &plds, &powt, lane, key);
+            else run_pair<1>(a, r, ho, &plds, &powt, lane, key);
+            forget42(p, s, o);
             __syncthreads();
             if (threadIdx.x == 0) pair_state = -1;
             __syncthreads();
@@ -1593,9 +1606,10 @@ void k_dop853_final42_resume(Final42Args a, ResumeArgs r) {
             if (!moved) traj = -1;
             const int tr = __builtin_amdgcn_readlane(traj, src);
             const double t0 = a.t0[tr];
-            run_wide(a, &powt, lane, src, traj, p, s,
+            run_wide(a, &powt, &rec[wid], &plds.zero[0], lane, src, traj, p, s,
                      SimdReserve{r.simd_tab, key, r.exclusive, lane, t0, a.tf[tr] - t0, false});
             if (lane == 0) atomicSub(&r.ctr[3], 1);
+            forget42(p, s, o);
             traj = -1;
             continue;
         }

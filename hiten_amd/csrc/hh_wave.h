@@ -1,24 +1,33 @@
-/* hh_wave.h -- one 42-d variational trajectory per wave (64 lanes).
+/* hh_wave.h -- one 42-d variational trajectory per wave (64 lanes), and the
+ * lane layout it shares with the two-wave form (hh_pair.h).
  *
- * Lane L = 8*b + d holds entry d (0..5) of block b (0..6) of the 42-d state,
- * the blocks being those of Lane42 (b = 0: the state x, b = 1..6: STM column
- * b-1); lanes with d > 5 or b = 7 are idle.  Every per-component expression
- * is Lane42's (and so the reference's, dynamics/rtbp.py:115-141, 219-242 and
- * integrators/rk.py:1636-1699, 1836-1874, 2457-2484), evaluated one component
- * per lane instead of six, so results are bit-identical to Lane42's.  What
- * the wave shares is formed once, in parallel lanes:
- *   - the twelve quotients of the variational field, one per lane 0..11,
- *     then read back as wave-uniform values;
- *   - the three pow calls of the step-size controller, in lanes 0..2;
- *   - the error-norm block sums, each formed in Lane42's in-lane order and
+ * Lanes 0..15 (the wave's first DPP row) hold the state: x, y, z in lanes
+ * 0..2, vx, vy, vz in lanes 4..6, the constant 1 in lane 3, 0 in lane 7.
+ * Lanes 16 + 8 j .. hold STM column j (j = 0..5) the same way: entries 0..2,
+ * 0, entries 3..5, 0.  Every per-component expression is Lane42's (and so the
+ * reference's, dynamics/rtbp.py:115-141, 219-242 and integrators/rk.py:
+ * 1636-1699, 1836-1874, 2457-2484), evaluated one component per lane instead
+ * of six, so results are bit-identical to Lane42's:
+ *   - the twelve quotients of the variational field are formed one per lane
+ *     in lanes 4..15, each lane raising its own primary's distance to the
+ *     power its quotient needs;
+ *   - the state's rows take theirs by DPP; the columns read the other six and
+ *     the coordinates from LDS, where the first row writes them;
+ *   - the three pow calls of the step-size controller run in lanes 0..2;
+ *   - the error-norm block sums are formed in Lane42's in-lane order and
  *     combined by the same block tree.
- * The per-attempt instruction stream is about a third of Lane42's, which is
- * what bounds a trajectory that runs alone on its SIMD.
+ *
+ * What bounds a trajectory that runs alone on its SIMD is the length of its
+ * wave's instruction stream (about 5 cycles an instruction) and the latency
+ * of the state's chain, so an attempt is branch-free on the unscaled forms of
+ * hh_fast.h and is evaluated again with the general ones if a value leaves
+ * their range.
  */
 #ifndef HH_WAVE_H
 #define HH_WAVE_H
 
 #include "hh_device.h"
+#include "hh_group6.h"
 
 namespace hh {
 
@@ -33,167 +42,234 @@ __device__ __forceinline__ double xor_sign(double v, unsigned long long s) {
     return __longlong_as_double(__double_as_longlong(v) ^ (long long)s);
 }
 
-struct Wave42 {
+/* What the state's row hands to the columns in one right-hand side: every
+ * lane's quotient and distance component (those of lanes 4..15 are read).
+ * Lanes whose row of F has no entries read a record of zeros.             */
+struct StageRec {
+    double q[64], u[64];
+};
+
+/* Lane layout, constants and the two halves of the field */
+struct Var42 {
     double mu, mu2;
     int lane;
-    int d;                    /* entry within the block                          */
-    bool st;                  /* block 0                                         */
-    bool act;                 /* holds a component (b < 7, d < 6)               */
-    bool odd;                 /* quotient lane on the second primary's side      */
-    int kind;                 /* quotient kind of lanes 0..11                    */
-    int pv_addr;              /* ds_bpermute byte address of the lane holding the
-                                 velocity-part entry this lane's row needs       */
-    double cl;                /* mu (even lanes) or -mu2 (odd lanes): x + cl is
-                                 x + mu or x - mu2 exactly                       */
+    int l;                    /* lane & 7                                        */
+    int d;                    /* entry 0..5 of the block, 6 or 7 without one      */
+    bool act;                 /* holds a component                               */
+    bool st;                  /* in the state's row                              */
+    bool vel;                 /* in a quad of velocity entries                   */
+    bool xy;                  /* lane of vx or vy of the state                   */
+    bool p5;                  /* this lane's quotient divides by r^5             */
+    bool quot;                /* holds a quotient (lanes 4..15)                  */
+    double cl;                /* x + cl: the lane's primary's x distance          */
+    double b;                 /* w + b: the lane's distance component             */
+    double cm, ca;            /* numerator cm (w + b) + ca                       */
+    double ka, kb;            /* mu2, mu in the state's velocity lanes, else 0   */
+    double c2;                /* factor of the velocity entry: state rows         */
+    double e2;                /* and column rows                                 */
+    double diag;              /* 1, 1, 0: the constant of the Hessian's diagonal */
     unsigned long long sign;  /* bit 63: this lane's derivative is negated       */
     const PowTab* pt;         /* hh_pow's tables (an LDS copy)                   */
+    DopRow tab;               /* tableau coefficients, one copy per row           */
 
     __device__ __forceinline__ void setup(int lane_, double mu_, int fwd,
                                           unsigned long long flip, const PowTab* pt_) {
         lane = lane_;
         pt = pt_;
-        const int b = lane >> 3;
-        d = lane & 7;
-        st = (b == 0);
-        act = (b < 7) && (d < 6);
-        odd = (lane & 1) != 0;
-        kind = (lane >> 1) % 6;
+        l = lane & 7;
+        st = lane < 16;
+        act = l != 3 && l != 7 && (lane < 8 || !st);
+        vel = (l & 4) != 0;
+        d = l < 3 ? l : (l == 3 ? 6 : (l < 7 ? l - 1 : 7));
+        xy = lane == 4 || lane == 5;
+        quot = st && lane >= 4;
+        p5 = lane >= 8 && lane < 12;
         mu = mu_;
         mu2 = 1.0 - mu_;
-        const int c = act ? comp42(b, d) : 0;
-        sign = (act && fwd == -1 && ((flip >> c) & 1ULL)) ? (1ULL << 63) : 0ULL;
-        /* rows 0..2 need entry d+3; row 3 needs entry 4 and row 4 entry 3
-         * (Coriolis terms of the column rows and of the state rows)          */
-        const int src = (d < 3) ? d + 3 : ((d == 3) ? 4 : 3);
-        pv_addr = ((lane & ~7) | src) << 2;
-        cl = odd ? -mu2 : mu_;
+        const bool second = lane >= 10 && st;
+        cl = second ? -mu2 : mu_;
+        /* lanes   4 xm/r3   5 y/r3        6 z/r3   7 mu2/r3
+         *         8 mu2/r5  9 (mu2 xm)/r5 10 mu/R5 11 (mu xr)/R5
+         *        12 xr/R3  13 y/R3       14 z/R3  15 mu/R3
+         * from w = x, y, z, 1 in lanes 4..7 and 12..15, x in lanes 8..11;
+         * adding -0.0 leaves every value, signed zeros too, as it is       */
+        b = (lane == 4 || lane == 9) ? mu_ : ((lane == 11 || lane == 12) ? -mu2 : -0.0);
+        const double m = second ? mu_ : mu2;
+        cm = (lane == 7 || lane == 9 || lane == 11 || lane == 15)
+                 ? m : ((quot && lane != 8 && lane != 10) ? 1.0 : 0.0);
+        ca = (lane == 8 || lane == 10) ? m : (lane < 4 ? 0.0 : -0.0);
+        const bool sv = lane >= 4 && lane < 7;
+        ka = sv ? mu2 : 0.0;
+        kb = sv ? mu_ : 0.0;
+        /* lane 6 multiplies lane 7's zero: -0.0, which adds nothing        */
+        c2 = lane < 4 ? 1.0 : (lane == 4 ? 2.0 : (lane == 5 ? -2.0 : (lane == 6 ? -1.0 : 0.0)));
+        e2 = l < 3 ? 1.0 : (l == 4 ? 2.0 : (l == 5 ? -2.0 : 0.0));
+        diag = (l == 4 || l == 5) ? 1.0 : 0.0;
+        sign = (act && fwd == -1 && ((flip >> comp()) & 1ULL)) ? (1ULL << 63) : 0ULL;
+        tab.fill(lane);
     }
 
-    /* accessors shared with the pair layout */
-    __device__ __forceinline__ bool holds() const { return act; }
-    __device__ __forceinline__ bool leader() const { return lane == 0; }
-    __device__ __forceinline__ int comp() const { return comp42(lane >> 3, d); }
+    /* Lane42's block (0 the state, 1..6 the columns) and the component's place
+     * in the 42-vector, of a lane that holds one                            */
+    __device__ __forceinline__ int block() const { return st ? 0 : (lane >> 3) - 1; }
+    __device__ __forceinline__ int comp() const { return comp42(block(), d < 6 ? d : 0); }
+    /* what lanes without a component hold */
+    __device__ __forceinline__ double idle() const { return lane == 3 ? 1.0 : 0.0; }
 
-    __device__ __forceinline__ double gather_pv(double v) const {
-        const int lo = __builtin_amdgcn_ds_bpermute(pv_addr, __double2loint(v));
-        const int hi = __builtin_amdgcn_ds_bpermute(pv_addr, __double2hiint(v));
-        return __hiloint2double(hi, lo);
+    /* the velocity entry of this lane's row: lanes 0..2 of a half row take
+     * lanes 4..6, lane 4 lane 5, lane 5 lane 4, lane 6 lane 7's zero        */
+    __device__ __forceinline__ double vel_entry(double v) const {
+        return dpp_into<DPP_SHL4, BANKS_POS>(quad_get<QUAD_SWAP01>(v), v);
     }
 
-    /* derivative of this lane's component; v = this lane's component of the
-     * stage state (idle lanes: any finite value)                            */
-    __device__ __forceinline__ double rhs(double v) const {
-        const double p0 = group_get<0>(v);
-        const double p1 = group_get<1>(v);
-        const double p2 = group_get<2>(v);
-        const double pv = gather_pv(v);
-        const double x = rlane(v, 0);
-        const double y = rlane(v, 1);
-        const double z = rlane(v, 2);
-        const double xm = x + mu;
-        const double xr = x - mu2;
-        /* quotient lane k = kind*2 + odd (Lane42's q1..q6 of both lane kinds):
-         *  k: 0 xm/r3  1 xr/R3  2 y/r3  3 y/R3  4 z/r3  5 z/R3
-         *     6 mu2/r5 7 mu/R5  8 mu2/r3 9 mu/R3 10 (mu2 xm)/r5 11 (mu xr)/R5 */
+    /* This lane's quotient of the field, from the state in lanes 0..7 of v;
+     * w and u as in setup's table.                                          */
+    template <bool FAST>
+    __device__ __forceinline__ double quotient(double v, FastChk& c, double& w,
+                                               double& u) const {
+        const double x = row_bcast<0>(v);
+        const double y = row_bcast<1>(v);
+        const double z = row_bcast<2>(v);
+        w = dpp_into<0x11C, 0x8>(dpp_into<DPP_SHR4, 0x2>(x, v), v);   /* row_shr 12, 4 */
+        u = w + b;
+        const double num = __builtin_fma(cm, u, ca);
         const double xo = x + cl;
         const double P = (xo * xo + y * y) + z * z;
-        double P3, P5;
-        hh_dev_pow15_25(P, &P3, &P5);
-        const double m = odd ? mu : mu2;
-        double num = xo;
-        num = (kind == 1) ? y : num;
-        num = (kind == 2) ? z : num;
-        num = (kind == 3 || kind == 4) ? m : num;
-        num = (kind == 5) ? m * xo : num;
-        const double q = num / ((kind == 3 || kind == 5) ? P5 : P3);
-        const double Q0 = rlane(q, 0), Q1 = rlane(q, 1), Q2 = rlane(q, 2), Q3 = rlane(q, 3);
-        const double Q4 = rlane(q, 4), Q5 = rlane(q, 5), Q6 = rlane(q, 6), Q7 = rlane(q, 7);
-        const double Q8 = rlane(q, 8), Q9 = rlane(q, 9), Q10 = rlane(q, 10), Q11 = rlane(q, 11);
-        /* state rows (rtbp.py:233-242); pv is vy on lane 3, vx on lane 4 */
-        const double s3 = ((x - mu2 * Q0) - mu * Q1) + 2.0 * pv;
-        const double s4 = ((y - mu2 * Q2) - mu * Q3) - 2.0 * pv;
-        const double s5 = (-mu2 * Q4) - mu * Q5;
-        /* Hessian entries (rtbp.py:124-141) */
+        if constexpr (FAST) {
+            c.dist(P);
+            c.num(u);
+            /* fast_pow15_25 for the one power this lane needs:
+             * base * s with base = P or P^2 (= base + be), t = s or P s      */
+            double s, h;
+            fast_root(P, s, h);
+            const double e = __builtin_fma(-s, s, P);
+            const double he = 0.5 * e;
+            const double q = P * P, qe = __builtin_fma(P, P, -q);
+            const double base = p5 ? q : P, be = p5 ? qe : 0.0;
+            const double t = (p5 ? P : 1.0) * s;
+            const double p = base * s, pe = __builtin_fma(base, s, -p);
+            const double D = p + (pe + (t * he + be * s));
+            const double h2 = h * h;
+            const double y15 = (8.0 * h) * h2;
+            const double R = rcp_step(D, y15 * (p5 ? 4.0 * h2 : 1.0));
+            return fast_div(num, D, R);
+        } else {
+            double P3, P5;
+            hh_dev_pow15_25(P, &P3, &P5);
+            const double q = num / (p5 ? P5 : P3);
+            return quot ? q : 0.0;
+        }
+    }
+
+    /* derivative of this lane's state component (rtbp.py:233-242):
+     * rows 0..2  the velocity entry
+     * row 3      ((x - mu2 xm/r3) - mu xr/R3) + 2 vy
+     * row 4      ((y - mu2 y/r3) - mu y/R3) - 2 vx
+     * row 5      (-mu2 z/r3) - mu z/R3
+     * all as ((w0 - ka q) - kb q2) + c2 pv                                  */
+    template <bool FAST>
+    __device__ __forceinline__ double state_row(double v, double q, double w) const {
+        const double pv = vel_entry(v);
+        const double q2 = dpp_into<0x108, 0x2>(0.0, q);   /* row_shl 8 into lanes 4..7 */
+        const double w0 = xy ? w : -0.0;
+        const double o = ((w0 - ka * q) - kb * q2) + c2 * pv;
+        if constexpr (FAST) return o;
+        return (act && st) ? o : 0.0;
+    }
+
+    /* derivative of this lane's column entry: row d of F @ Phi[:, j]
+     * (rtbp.py:124-141, column_rhs); r: the stage's record in velocity lanes,
+     * zeros in the others                                                   */
+    template <bool FAST>
+    __device__ __forceinline__ double column_row(double v, const StageRec& r) const {
+        const int row = vel ? (l & 3) : 0;
+        const double pv = vel_entry(v);
+        const double t = dpp_into<DPP_SHR4, BANKS_VEL>(v, v);
+        const double p0 = quad_get<0x00>(t), p1 = quad_get<0x55>(t), p2 = quad_get<0xAA>(t);
+        const double Q6 = r.q[8], Q7 = r.q[10], Q8 = r.q[7], Q9 = r.q[15];
+        const double Q10 = r.q[9], Q11 = r.q[11];
+        const double y = r.u[5], z = r.u[6];
+        const double pa = r.u[4 + row], pb = r.u[12 + row];   /* xm, y, z and xr, y, z */
         const double a53 = Q6 * 3.0;
         const double b53 = Q7 * 3.0;
         const double c3 = Q8 + Q9;
         const double gx = Q10 + Q11;
-        const double uxx = ((1.0 + a53 * (xm * xm)) + b53 * (xr * xr)) - c3;
-        const double uyy = ((1.0 + a53 * (y * y)) + b53 * (y * y)) - c3;
-        const double uzz = ((0.0 + a53 * (z * z)) + b53 * (z * z)) - c3;
+        const double dd = ((diag + a53 * (pa * pa)) + b53 * (pb * pb)) - c3;
         const double uxy = (3.0 * y) * gx;
         const double uxz = (3.0 * z) * gx;
         const double uyz = ((3.0 * y) * z) * (Q6 + Q7);
-        /* row d of F @ Phi[:, j] (column_rhs) */
-        const double cA = (d == 3) ? uxx : ((d == 4) ? uxy : uxz);
-        const double cB = (d == 3) ? uxy : ((d == 4) ? uyy : uyz);
-        const double cC = (d == 3) ? uxz : ((d == 4) ? uyz : uzz);
+        const double cA = (l == 4) ? dd : ((l == 5) ? uxy : uxz);
+        const double cB = (l == 4) ? uxy : ((l == 5) ? dd : uyz);
+        const double cC = (l == 4) ? uxz : ((l == 5) ? uyz : dd);
         const double acc = ((0.0 + cA * p0) + cB * p1) + cC * p2;
-        const double E = (d == 3) ? 2.0 : -2.0;
-        const double row = (d == 5) ? acc : acc + E * pv;
-        const double sv = (d == 3) ? s3 : ((d == 4) ? s4 : s5);
-        const double lo3 = st ? pv : (0.0 + pv);
-        const double hi3 = st ? sv : row;
-        return xor_sign((d < 3) ? lo3 : hi3, sign);
+        const double o = acc + e2 * pv;
+        if constexpr (FAST) return o;
+        return vel ? (l == 7 ? 0.0 : o) : (l == 3 ? 0.0 : 0.0 + pv);
     }
 
-    /* Lane42::reduce of in-lane sums over a block: sq = this lane's term */
-    __device__ __forceinline__ double block_tree(double sq) const {
-        const double g0 = group_get<0>(sq);
-        const double g1 = group_get<1>(sq);
-        const double g2 = group_get<2>(sq);
-        const double g3 = group_get<3>(sq);
-        const double g4 = group_get<4>(sq);
-        const double g5 = group_get<5>(sq);
-        const double blk = (((((0.0 + g0) + g1) + g2) + g3) + g4) + g5;
-        const double B0 = rlane(blk, 0), B1 = rlane(blk, 8), B2 = rlane(blk, 16);
-        const double B3 = rlane(blk, 24), B4 = rlane(blk, 32), B5 = rlane(blk, 40);
-        const double B6 = rlane(blk, 48);
-        return ((B0 + B1) + (B2 + B3)) + ((B4 + B5) + (B6 + 0.0));
+    /* Lane42's in-lane sum over a block (entries 0..5 from 0.0), in the lane
+     * of entry 5: the running sum moves from lane to lane                  */
+    __device__ __forceinline__ static double block_sum(double term) {
+        double s = 0.0 + term;
+        s = row_shr<1>(s) + term;
+        s = row_shr<1>(s) + term;
+        s = row_shr<2>(s) + term;
+        s = row_shr<1>(s) + term;
+        return row_shr<1>(s) + term;
     }
+    template <int N>
+    __device__ __forceinline__ static double row_shr(double v) {
+        return dpp_into<0x110 + N, 0xF>(v, v);
+    }
+    static constexpr int SUM_LANE0 = 6;                    /* the state's block sum */
+    __device__ __forceinline__ static constexpr int sum_lane(int blk) { return 8 * blk + 14; }
 
-    /* dop853_attempt, one component per lane */
-    __device__ __forceinline__ double attempt(double y, double (&k)[DOP_K], double h, double rtol,
-                                              double atol, double& yh) const {
-#pragma unroll
-        for (int i = 1; i < DOP_S; ++i) {
-            double ys = y;
-#pragma unroll
-            for (int j = 0; j < i; ++j) {
-                const double a = HH_DOP_A[i][j];
-                if (a != 0.0) {
-                    const double ha = h * a;
-                    ys = ys + ha * k[j];
-                }
-            }
-            k[i] = rhs(ys);
-        }
-        yh = y;
-#pragma unroll
-        for (int j = 0; j < DOP_S; ++j) {
-            const double bb = HH_DOP_B[j];
-            if (bb != 0.0) {
-                const double hb = h * bb;
-                yh = yh + hb * k[j];
-            }
-        }
-        k[DOP_S] = rhs(yh);
+    /* scaled errors of this lane's component (rk.py:2457-2463), 0 without one */
+    template <bool FAST>
+    __device__ __forceinline__ void scaled_errors(double y, double yh, const double (&k)[DOP_K],
+                                                  double h, double rtol, double atol,
+                                                  FastChk& c, double& q5, double& q3) const {
         double e5 = 0.0, e3 = 0.0;
+        int n = 0;
 #pragma unroll
-        for (int j = 0; j < DOP_K; ++j) {
-            const double c5 = HH_DOP_E5[j];
-            const double c3 = HH_DOP_E3[j];
-            if (c5 != 0.0) e5 = e5 + c5 * k[j];
-            if (c3 != 0.0) e3 = e3 + c3 * k[j];
+        for (int j = 0; j < DOP_K; ++j)
+            if (HH_DOP_E5[j] != 0.0) e5 = e5 + tab.e.at(n++) * k[j];
+#pragma unroll
+        for (int j = 0; j < DOP_K; ++j)
+            if (HH_DOP_E3[j] != 0.0) e3 = e3 + tab.e.at(n++) * k[j];
+        const double m = np_max(__builtin_fabs(y), __builtin_fabs(yh));
+        const double sc = act ? atol + rtol * m : 1.0;
+        const double n5 = act ? e5 * h : 0.0;
+        const double n3 = act ? e3 * h : 0.0;
+        if constexpr (FAST) {
+            c.scale(sc);
+            c.num(n5);
+            c.num(n3);
+            const double r = fast_rcp(sc);
+            q5 = fast_div(n5, sc, r);
+            q3 = fast_div(n3, sc, r);
+        } else {
+            q5 = n5 / sc;
+            q3 = n3 / sc;
         }
-        const double sc = atol + rtol * np_max(__builtin_fabs(y), __builtin_fabs(yh));
-        const double q5 = (e5 * h) / sc;
-        const double q3 = (e3 * h) / sc;
-        const double s5 = block_tree(q5 * q5);
-        const double s3 = block_tree(q3 * q3);
-        if (s5 == 0.0 && s3 == 0.0) return 0.0;
-        const double denom = s5 + 0.01 * s3;
-        return (__builtin_fabs(h) * s5) / __builtin_sqrt(denom * 42.0);
+    }
+
+    /* error norm from the two sums of squares (rk.py:2464-2467) */
+    template <bool FAST>
+    __device__ __forceinline__ static double error_norm(double s5, double s3, double h,
+                                                        FastChk& c) {
+        const double denom = (s5 + 0.01 * s3) * 42.0;
+        const double top = __builtin_fabs(h) * s5;
+        if constexpr (FAST) {
+            c.scale(denom);
+            c.num(top);
+            double g;
+            const double r = fast_sqrt(denom, g);
+            return fast_div(top, r, rcp_step(r, g + g));
+        } else {
+            if (s5 == 0.0 && s3 == 0.0) return 0.0;
+            return top / __builtin_sqrt(denom);
+        }
     }
 
     /* pi_accept_factor(err, err_prev) and pi_reject_factor(err) with their
@@ -221,48 +297,185 @@ struct Wave42 {
         if (g > 10.0) g = 10.0;
         f_rej = g;
     }
+};
 
-    /* dense-output value at tf of the step [t, t + hs] (FinalOut::accepted) */
-    __device__ __forceinline__ double dense_at(double y_old, double y_new, const double (&k)[DOP_K],
-                                               double hs, double xq) const {
-        double kx[DOP_SX - DOP_K];
+/* dop853_attempt's stages and solution, one component per lane; W supplies
+ * the right-hand side of stage i (rhs_form<FAST, i % 2>)                   */
+template <bool FAST, class W>
+__device__ __forceinline__ double dop853_stages(const W& w, double y, double (&k)[DOP_K], double h,
+                                                FastChk& c) {
+    const RowTab<58> ha = w.tab.a.times(h);
+    int n = 0;
 #pragma unroll
-        for (int sr = DOP_K; sr < DOP_SX; ++sr) {
-            double acc = 0.0;
+    for (int i = 1; i < DOP_S; ++i) {
+        double ys = y;
 #pragma unroll
-            for (int r = 0; r < sr; ++r) {
-                const double a = HH_DOP_A[sr][r];
-                if (a != 0.0) acc = acc + a * (r < DOP_K ? k[r] : kx[r - DOP_K]);
-            }
-            kx[sr - DOP_K] = rhs(y_old + hs * acc);
+        for (int j = 0; j < i; ++j)
+            if (HH_DOP_A[i][j] != 0.0) ys = ys + ha.at(n++) * k[j];
+        k[i] = (i % 2 == 0) ? w.template rhs_form<FAST, 0>(ys, c)
+                            : w.template rhs_form<FAST, 1>(ys, c);
+    }
+    double yh = y;
+#pragma unroll
+    for (int j = 0; j < DOP_S; ++j)
+        if (HH_DOP_B[j] != 0.0) yh = yh + ha.at(n++) * k[j];
+    k[DOP_S] = w.template rhs_form<FAST, 0>(yh, c);
+    return yh;
+}
+
+/* The three extension stages and the seven interpolant rows of this lane's
+ * component (rk.py:1836-1874)                                              */
+template <class W>
+__device__ __forceinline__ void dop853_rows(const W& w, double y_old, double y_new,
+                                            const double (&k)[DOP_K], double hs,
+                                            double (&row)[DOP_P]) {
+    double kx[DOP_SX - DOP_K];
+#pragma unroll
+    for (int sr = DOP_K; sr < DOP_SX; ++sr) {
+        double acc = 0.0;
+#pragma unroll
+        for (int r = 0; r < sr; ++r) {
+            const double a = HH_DOP_A[sr][r];
+            if (a != 0.0) acc = acc + a * (r < DOP_K ? k[r] : kx[r - DOP_K]);
         }
-        const double omx = 1.0 - xq;
-        const double dy = y_new - y_old;
-        double v = 0.0;
+        const double ys = y_old + hs * acc;
+        kx[sr - DOP_K] = sr == DOP_K       ? w.template rhs<1>(ys)
+                         : sr == DOP_K + 1 ? w.template rhs<0>(ys)
+                                           : w.template rhs<2>(ys);
+    }
+    const double dy = y_new - y_old;
+    row[0] = dy;
+    row[1] = hs * k[0] - dy;
+    row[2] = 2.0 * dy - hs * (k[DOP_S] + k[0]);
 #pragma unroll
-        for (int i = DOP_P - 1; i >= 0; --i) {
-            double row;
-            if (i == 0) {
-                row = dy;
-            } else if (i == 1) {
-                row = hs * k[0] - dy;
-            } else if (i == 2) {
-                row = 2.0 * dy - hs * (k[DOP_S] + k[0]);
-            } else {
-                double acc = 0.0;
+    for (int i = 3; i < DOP_P; ++i) {
+        double acc = 0.0;
 #pragma unroll
-                for (int r = 0; r < DOP_SX; ++r) {
-                    const double c = HH_DOP_D[i - 3][r];
-                    if (c != 0.0) acc = acc + c * (r < DOP_K ? k[r] : kx[r - DOP_K]);
-                }
-                row = hs * acc;
-            }
-            v = v + row;
-            v = v * (((DOP_P - 1 - i) % 2 == 0) ? xq : omx);
+        for (int r = 0; r < DOP_SX; ++r) {
+            const double c = HH_DOP_D[i - 3][r];
+            if (c != 0.0) acc = acc + c * (r < DOP_K ? k[r] : kx[r - DOP_K]);
         }
-        return v + y_old;
+        row[i] = hs * acc;
+    }
+}
+
+/* zeros for the lanes that read none of the field's entries; a barrier of the
+ * workgroup must follow                                                     */
+__device__ __forceinline__ void wave_lds_clear(StageRec& zero) {
+    for (int i = (int)threadIdx.x; i < 64; i += (int)blockDim.x) {
+        zero.q[i] = 0.0;
+        zero.u[i] = 0.0;
+    }
+}
+
+struct Wave42 : Var42 {
+    StageRec* rec;            /* this wave's record                              */
+    const StageRec* mine;     /* what this lane reads: rec or the zeros          */
+
+    __device__ __forceinline__ void setup(int lane_, double mu_, int fwd,
+                                          unsigned long long flip, const PowTab* pt_,
+                                          StageRec* rec_, const StageRec* zero) {
+        Var42::setup(lane_, mu_, fwd, flip, pt_);
+        rec = rec_;
+        mine = (vel && l != 7) ? rec_ : zero;
+    }
+
+    /* accessors shared with the pair layout */
+    __device__ __forceinline__ bool holds() const { return act; }
+    __device__ __forceinline__ bool leader() const { return lane == 0; }
+
+    /* derivative of this lane's component; v = this lane's component of the
+     * stage state (idle() in lanes without one)                             */
+    template <bool FAST, int>
+    __device__ __forceinline__ double rhs_form(double v, FastChk& c) const {
+        double w, u;
+        const double q = quotient<FAST>(v, c, w, u);
+        rec->q[lane] = q;
+        rec->u[lane] = u;
+        /* the wave's own stores before its loads */
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const double os = state_row<FAST>(v, q, w);
+        const double oc = column_row<FAST>(v, *mine);
+        __builtin_amdgcn_wave_barrier();
+        return xor_sign(st ? os : oc, sign);
+    }
+
+    /* whether the state's lanes left the range of the unscaled forms */
+    __device__ __forceinline__ bool left_range(const FastChk& c) const {
+        return st && c.outside();
+    }
+
+    template <int BUF = 0>
+    __device__ __forceinline__ double rhs(double v) const {
+        FastChk c;
+        c.num(mu);
+        c.num(mu2);
+        const double o = rhs_form<true, BUF>(v, c);
+        if (__builtin_expect(__any(left_range(c)), 0)) return rhs_form<false, BUF>(v, c);
+        return o;
+    }
+
+    /* Lane42::reduce of in-lane sums over a block: sq = this lane's term */
+    __device__ __forceinline__ double block_tree(double sq) const {
+        const double s = block_sum(sq);
+        const double B0 = rlane(s, SUM_LANE0), B1 = rlane(s, sum_lane(1)), B2 = rlane(s, sum_lane(2));
+        const double B3 = rlane(s, sum_lane(3)), B4 = rlane(s, sum_lane(4));
+        const double B5 = rlane(s, sum_lane(5)), B6 = rlane(s, sum_lane(6));
+        return ((B0 + B1) + (B2 + B3)) + ((B4 + B5) + (B6 + 0.0));
+    }
+
+    /* initial_step (rk.py:2443-2448) with the block-tree sums of Lane42 */
+    __device__ __forceinline__ double initial_step(double y, double f0,
+                                                   const StepParams& sp) const {
+        const double sc = sp.atol + sp.rtol * __builtin_fabs(y);
+        const double ua = y / sc;
+        const double ub = f0 / sc;
+        const double s0 = block_tree(act ? ua * ua : 0.0);
+        const double s1 = block_tree(act ? ub * ub : 0.0);
+        const double sn = __builtin_sqrt(42.0);
+        return select_initial_step(__builtin_sqrt(s0) / sn, __builtin_sqrt(s1) / sn, sp.min_step,
+                                   sp.max_step);
+    }
+
+    template <bool FAST>
+    __device__ __forceinline__ double attempt_form(double y, double (&k)[DOP_K], double h,
+                                                   double rtol, double atol, double& yh,
+                                                   FastChk& cs, FastChk& ce) const {
+        yh = dop853_stages<FAST>(*this, y, k, h, cs);
+        double q5, q3;
+        scaled_errors<FAST>(y, yh, k, h, rtol, atol, ce, q5, q3);
+        const double s5 = block_tree(q5 * q5);
+        const double s3 = block_tree(q3 * q3);
+        return error_norm<FAST>(s5, s3, h, ce);
+    }
+
+    /* dop853_attempt, one component per lane */
+    __device__ __forceinline__ double attempt(double y, double (&k)[DOP_K], double h, double rtol,
+                                              double atol, double& yh) const {
+        FastChk cs, ce;
+        cs.num(mu);
+        cs.num(mu2);
+        double err = attempt_form<true>(y, k, h, rtol, atol, yh, cs, ce);
+        if (__builtin_expect(__any(left_range(cs) || ce.outside() || !(err < __builtin_inf())),
+                             0)) {
+            asm volatile("" : "+v"(h));
+            err = attempt_form<false>(y, k, h, rtol, atol, yh, cs, ce);
+        }
+        return err;
     }
 };
+
+/* dense_from_rows of the last step of an integration (FinalOut::accepted) */
+template <class W>
+__device__ __forceinline__ double dop853_dense_at(const W& w, double y_old, double y_new,
+                                                  const double (&k)[DOP_K], double hs,
+                                                  double xq) {
+    double row[DOP_P];
+    dop853_rows(w, y_old, y_new, k, hs, row);
+    return dense_from_rows(row, y_old, xq);
+}
 
 }  // namespace hh
 

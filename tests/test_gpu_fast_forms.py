@@ -1,7 +1,7 @@
 """GPU: the field and the step loops at the edges of the exponent range in
 which divisions and powers take their unscaled forms (squared distances in
 [2^-100, 2^100), coordinates and masses 0 or at least 2^-301, error scales in
-[2^-300, 2^300)), against the oracle bit for bit: states inside, on either
+[2^-300, 2^960)), against the oracle bit for bit: states inside, on either
 side of each bound, and both in one wave."""
 
 import numpy as np
@@ -76,6 +76,27 @@ def test_integration_at_the_range_bounds(gpu, oracle, dim, variant, n):
         assert np.array_equal(r.n_accepted.cpu().numpy(), na)
         assert np.array_equal(r.n_rejected.cpu().numpy(), nr)
         assert np.array_equal(r.status.cpu().numpy(), st)
+
+
+@pytest.mark.parametrize("variant", ["plain", "wide", "pair", "persistent", "persistent_pair"])
+def test_error_scales_at_their_bounds(gpu, oracle, variant):
+    """STMs that start large enough for the error scale rtol |Phi| to lie on
+    either side of 2^960, and small enough for entries below 2^-301."""
+    n = 24
+    rng = np.random.default_rng(3)
+    y0 = W.with_identity_stm(W.planar_seeds(rng, n))
+    size = 2.0 ** rng.permutation(np.array([0, 300, 500, 900, 998, 999, 1000, 1001, 1010, 1020,
+                                            -200, -300, -301, -302, -500, -1000] + [0] * 8))
+    y0[:, :36] *= size[:, None]
+    y0[::3, 1] = 2.0 ** -310
+    mu = np.full(n, MU)
+    tf = rng.uniform(0.05, 0.4, n)
+    r = batch.dop853_final(mu, y0, 0.0, tf, dim=42, variant=variant, max_steps=300)
+    want, na, nr, st = oracle.batch_dop853_final(mu, y0, np.zeros(n), tf, max_steps=300)
+    assert np.array_equal(r.y.cpu().numpy(), want, equal_nan=True)
+    assert np.array_equal(r.n_accepted.cpu().numpy(), na)
+    assert np.array_equal(r.n_rejected.cpu().numpy(), nr)
+    assert np.array_equal(r.status.cpu().numpy(), st)
 
 
 @pytest.mark.parametrize("n", [3, 4096, 4097])
