@@ -270,6 +270,19 @@ def prepare_final(mu, y0, t0, tf, dim: int = 6, order: str = "span") -> FinalBat
                       torch.empty(n, **i32), torch.empty(n, **i32), torch.empty(n, **i32), perm)
 
 
+def _auto_variant(dim: int, n: int) -> str:
+    """Layout of a final-value batch the caller leaves open.  6-d: lane groups
+    up to 65,536 trajectories, one per lane beyond.  42-d: two waves per
+    trajectory up to 4,096, where they fill the GPU (STMs of dispersed halo
+    states, pair / work-stealing / plain: 0.47 / 1.05 / 1.21 ms at 256, 1.42 /
+    1.55 / 1.79 ms at 4,096, 2.36 / 1.49 / 1.92 ms at 8,192), work stealing
+    beyond (2.7 against 5.8 ms at 65,536; 52 against 97 ms for uneven planar
+    states, whose longest trajectories end in a wave of their own)."""
+    if dim == 6:
+        return "wide" if n <= 65536 else "plain"
+    return "pair" if n <= 4096 else "persistent"
+
+
 def launch_final(b: FinalBatch, *, rtol: float = 1e-12, atol: float = 1e-12,
                  max_step: float = 1e4, min_step: float = MIN_STEP,
                  max_steps: int = DEFAULT_MAX_STEPS, forward: int = 1, flip_indices=None,
@@ -277,12 +290,11 @@ def launch_final(b: FinalBatch, *, rtol: float = 1e-12, atol: float = 1e-12,
     """Enqueue hh_dop853_final on the stream (asynchronous).
 
     ``variant``: "plain", "persistent" (dim 42), "persistent_pair" (dim 42),
-    "wide", "pair" (dim 42), or "auto" ("wide" for dim 6 up to 65,536
-    trajectories, else "plain").
+    "wide", "pair" (dim 42), or "auto" (by dimension and count).
     """
     lib = _lib.load()
     if variant == "auto":
-        variant = "wide" if b.dim == 6 and b.n <= 65536 else "plain"
+        variant = _auto_variant(b.dim, b.n)
     var = {"plain": _lib.HH_VARIANT_PLAIN, "persistent": _lib.HH_VARIANT_PERSISTENT,
            "wide": _lib.HH_VARIANT_WIDE, "pair": _lib.HH_VARIANT_PAIR,
            "persistent_pair": _lib.HH_VARIANT_PERSISTENT_PAIR}[variant]
@@ -339,6 +351,8 @@ def dop853_final(mu, y0, t0, tf, *, dim: int = 6, rtol: float = 1e-12, atol: flo
     """Adaptive DOP853 to tf; the state returned is the dense-output value at tf
     (the last row of _propagate_dynsys(..., steps=2)).
     """
+    if variant == "auto":
+        variant = _auto_variant(dim, 1 if np.ndim(y0) < 2 else len(y0))
     b = prepare_final(mu, y0, t0, tf, dim,
                       order="span" if variant.startswith("persistent") else None)
     launch_final(b, rtol=rtol, atol=atol, max_step=max_step, min_step=min_step,

@@ -1033,6 +1033,71 @@ struct WideFinal {
     }
 };
 
+/* Output policy of wide_loop: GridOut, this lane's component of every point.
+ * The times and abscissae of 64 points are formed at once, one per lane.   */
+struct WideGrid {
+    double* out;          /* this lane's component of the trajectory's first point */
+    const double* teval;
+    bool holds;
+    int m, q, lane;
+    double t0, tf, step, delta;
+    bool zstep;
+
+    template <class WL>
+    __device__ __forceinline__ void init(const Final42Args& a, const WL& W, int traj, double t0_,
+                                         double tf_) {
+        holds = W.holds();
+        out = a.yout + (size_t)traj * a.m * 42 + (holds ? W.comp() : 0);
+        teval = a.teval;
+        m = a.m;
+        q = 0;
+        lane = W.lane;
+        t0 = t0_;
+        tf = tf_;
+        delta = tf - t0;
+        step = delta / (double)(m - 1);
+        zstep = (step == 0.0);
+    }
+    __device__ __forceinline__ double tq(int i) const {
+        if (teval) return teval[i];
+        if (i == m - 1) return tf;
+        if (zstep) return ((double)i / (double)(m - 1)) * delta + t0;
+        return (double)i * step + t0;
+    }
+    __device__ __forceinline__ void put(int i, double v) const {
+        if (holds) out[(size_t)i * 42] = v;
+    }
+    __device__ __forceinline__ void stop(double y) {
+        for (; q < m; ++q) put(q, y);
+    }
+    template <class WL>
+    __device__ __forceinline__ void accepted(const WL& W, double y, double yh,
+                                             const double (&k)[DOP_K], double t, double t_new,
+                                             double, bool last) {
+        if (q >= m || !(last || tq(q) < t_new)) return;
+        const double hs = t_new - t;
+        if (hs == 0.0) {
+            stop(y);
+            return;
+        }
+        double row[DOP_P];
+        dop853_rows(W, y, yh, k, hs, row);
+        while (q < m) {
+            const int i = q + lane;
+            const double ti = tq(i < m ? i : m - 1);
+            const double x = (ti - t) / hs;
+            /* the points up to the first one this step does not cover */
+            const unsigned long long no = ~__ballot(i < m && (last || ti < t_new));
+            const int cnt = no ? __ffsll((long long)no) - 1 : 64;
+#pragma unroll 4
+            for (int j = 0; j < cnt; ++j)
+                put(q + j, dense_from_rows(row, y, rlane(x, j)));
+            q += cnt;
+            if (cnt < 64) break;
+        }
+    }
+};
+
 /* traj_iterate for one trajectory in a wave-wide layout (Wave42 or Pair42),
  * from the current (y, k[0], t, h, err_prev, counters) to its end          */
 template <class WL, class Out, class Hook = NoHook>
@@ -1101,14 +1166,20 @@ __device__ __forceinline__ bool no_span(double t0, double tf) {
 
 /* the stores of store42 */
 template <class WL>
-__device__ __forceinline__ void wide_store(const Final42Args& a, const WL& W, int traj, double out,
-                                           int status, int nacc, int nrej) {
-    if (W.holds()) a.yout[(size_t)W.comp() * a.n + traj] = out;
+__device__ __forceinline__ void wide_counts(const Final42Args& a, const WL& W, int traj,
+                                            int status, int nacc, int nrej) {
     if (W.leader()) {
         if (a.status) a.status[traj] = status;
         if (a.nacc) a.nacc[traj] = nacc;
         if (a.nrej) a.nrej[traj] = nrej;
     }
+}
+
+template <class WL>
+__device__ __forceinline__ void wide_store(const Final42Args& a, const WL& W, int traj, double out,
+                                           int status, int nacc, int nrej) {
+    if (W.holds()) a.yout[(size_t)W.comp() * a.n + traj] = out;
+    wide_counts(a, W, traj, status, nacc, nrej);
 }
 
 /* wide_loop, then the stores of store42 */
@@ -1182,20 +1253,29 @@ __global__ __launch_bounds__(BLOCK) void k_dop853_final42_wide(Final42Args a) {
 /* One trajectory per pair of waves (128-thread workgroup) from the start:
  * the state wave and the STM wave of Pair42 side by side on two SIMDs.  Both
  * waves take the same branches and so meet the same barriers.               */
-template <int ROLE>
+template <bool GRID, int ROLE>
 __device__ __forceinline__ void pair_from_start(const Final42Args& a, PairLds* lds,
                                                 const PowTab* pt, int traj, int lane) {
     Pair42<ROLE> P;
     P.setup(lane, a.mu[traj], a.fwd, a.flip, lds, pt);
     const double y0 = P.holds() ? a.y0[(size_t)P.comp() * a.n + traj] : P.idle();
     const double t0 = a.t0[traj], tf = a.tf[traj];
-    WideFinal o;
     int status = ST_OK, nacc = 0, nrej = 0;
-    o.stop(y0);
-    if (!no_span(t0, tf)) wide_from_start(a.sp, P, y0, t0, tf, o, status, nacc, nrej);
-    wide_store(a, P, traj, o.v, status, nacc, nrej);
+    if constexpr (GRID) {
+        WideGrid o;
+        o.init(a, P, traj, t0, tf);
+        if (no_span(t0, tf)) o.stop(y0);
+        else wide_from_start(a.sp, P, y0, t0, tf, o, status, nacc, nrej);
+        wide_counts(a, P, traj, status, nacc, nrej);
+    } else {
+        WideFinal o;
+        o.stop(y0);
+        if (!no_span(t0, tf)) wide_from_start(a.sp, P, y0, t0, tf, o, status, nacc, nrej);
+        wide_store(a, P, traj, o.v, status, nacc, nrej);
+    }
 }
 
+template <bool GRID>
 __global__ __launch_bounds__(128) void k_dop853_final42_pair(Final42Args a) {
     __shared__ PairLds lds;
     __shared__ PowTab powt;
@@ -1207,9 +1287,9 @@ __global__ __launch_bounds__(128) void k_dop853_final42_pair(Final42Args a) {
     if (traj >= a.n) return;
     /* the role in a scalar register: the branch is a uniform one */
     if (__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) == 0)
-        pair_from_start<0>(a, &lds, &powt, traj, lane);
+        pair_from_start<GRID, 0>(a, &lds, &powt, traj, lane);
     else
-        pair_from_start<1>(a, &lds, &powt, traj, lane);
+        pair_from_start<GRID, 1>(a, &lds, &powt, traj, lane);
 }
 
 /* A wave that has handed its trajectories on forgets them: their registers are
@@ -2118,7 +2198,7 @@ int hh_dop853_final(int n, int dim, const double* mu, const double* t0, const do
         return check_launch("hh_dop853_final(42, plain) launch");
     }
     if (variant == HH_VARIANT_PAIR) {
-        hipLaunchKernelGGL(k_dop853_final42_pair, dim3(n), dim3(128), 0, st, a);
+        hipLaunchKernelGGL(k_dop853_final42_pair<false>, dim3(n), dim3(128), 0, st, a);
         return check_launch("hh_dop853_final(42, pair) launch");
     }
     if (variant == HH_VARIANT_WIDE) {
@@ -2246,6 +2326,14 @@ int hh_dop853_final_static(int n, int dim, const double* mu, const double* t0, c
                            need > 0 ? STATIC_SCRATCH_BYTES : 0, order, stream);
 }
 
+/* Up to this many 42-d trajectories a grid is formed one trajectory per
+ * two-wave workgroup (Pair42, two waves a SIMD), more one per 8-lane group
+ * (Lane42).  Pair against lanes, halo orbits over a period: one orbit x 1,000
+ * points 0.43 and 1.33 ms, 200 x 200 points 0.47 and 1.11 ms, 1,024 x 2
+ * points 0.48 and 0.65 ms, 1,024 x 1,000 0.70 and 1.79 ms; 2,048 x 2 points
+ * 0.89 and 0.66 ms, 2,048 x 1,000 1.38 and 1.78 ms.                         */
+constexpr int PAIR_GRID_MAX = 1024;
+
 int hh_dop853_grid(int n, int dim, const double* mu, const double* t0, const double* tf, int m,
                    const double* t_eval, double rtol, double atol, double max_step,
                    double min_step, long long max_steps, int fwd, unsigned long long flip_mask,
@@ -2280,13 +2368,18 @@ int hh_dop853_grid(int n, int dim, const double* mu, const double* t0, const dou
     a.y0 = y0; a.yout = out; a.status = status; a.nacc = n_acc; a.nrej = n_rej; a.m = m;
     a.teval = t_eval;
     if (block <= 0) block = 256;
+    if (block != 64 && block != 128 && block != 256 && block != 512)
+        return fail(HH_ERR_ARGS, "hh_dop853_grid: block must be 64, 128, 256 or 512");
+    if (n <= PAIR_GRID_MAX) {
+        hipLaunchKernelGGL(k_dop853_final42_pair<true>, dim3(n), dim3(128), 0, st, a);
+        return check_launch("hh_dop853_grid(42, pair) launch");
+    }
     const int g = blocks_for((long long)n * 8, block);
     switch (block) {
         case 64: hipLaunchKernelGGL((k_dop853_final42_plain<64, true>), dim3(g), dim3(64), 0, st, a); break;
         case 128: hipLaunchKernelGGL((k_dop853_final42_plain<128, true>), dim3(g), dim3(128), 0, st, a); break;
         case 256: hipLaunchKernelGGL((k_dop853_final42_plain<256, true>), dim3(g), dim3(256), 0, st, a); break;
-        case 512: hipLaunchKernelGGL((k_dop853_final42_plain<512, true>), dim3(g), dim3(512), 0, st, a); break;
-        default: return fail(HH_ERR_ARGS, "hh_dop853_grid: block must be 64, 128, 256 or 512");
+        default: hipLaunchKernelGGL((k_dop853_final42_plain<512, true>), dim3(g), dim3(512), 0, st, a); break;
     }
     return check_launch("hh_dop853_grid(42) launch");
 }

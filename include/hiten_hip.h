@@ -217,8 +217,10 @@ int hh_dop853_final_static(int n, int dim, const double* mu, const double* t0, c
  * numpy.isclose calls zero repeats y0 (dynamics/base.py:421-424).
  *   out : [n][m][dim] (trajectory-major, the reference's (steps, dim)
  *         array per trajectory)
- *   variant : HH_VARIANT_PLAIN, or HH_VARIANT_WIDE for dim 6 (one
- *         trajectory per 8-lane group, one component per lane)           */
+ *   variant : HH_VARIANT_PLAIN (dim 6: one trajectory per lane; dim 42: one
+ *         per two-wave workgroup up to 1,024 trajectories, one per 8-lane
+ *         group beyond), or HH_VARIANT_WIDE for dim 6 (one trajectory per
+ *         lane group, one component per lane); same results either way   */
 int hh_dop853_grid(int n, int dim, const double* mu, const double* t0, const double* tf, int m,
                    const double* t_eval, double rtol, double atol, double max_step,
                    double min_step, long long max_steps, int fwd, unsigned long long flip_mask,

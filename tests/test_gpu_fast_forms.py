@@ -125,3 +125,53 @@ def test_lane_groups_on_either_side_of_their_size_rule(gpu, n):
                                                **kw)).values())
         same(lambda v: vars(batch.dop853_event(MU, y, 0.0, tf, variant=v, ev_index=5,
                                                direction=1, **kw)).values())
+
+
+@pytest.mark.parametrize("n,m", [(1, 2), (3, 130), (1024, 65), (1025, 65)])
+def test_stm_grids_on_either_side_of_their_size_rule(gpu, oracle, n, m):
+    """42-d grids up to 1,024 trajectories (two waves each) and beyond (lane
+    groups): every point of sampled trajectories against the oracle, its end
+    against the end-state kernels; more and fewer points than the 64 a wave
+    forms at once, several in one step, shared output times, a zero span, an
+    attempt limit, backward."""
+    rng = np.random.default_rng(n)
+    x = W.planar_seeds(rng, n)
+    y0 = W.with_identity_stm(x)
+    tf = rng.uniform(0.3, 1.2, n)
+    tf[n // 2] = 0.0
+    flip = slice(36, 42)
+    t_eval = np.sort(rng.uniform(0.0, 0.7, m))
+    t_eval[0] = 0.0
+    some = sorted({0, n // 2, n - 1})
+    for fwd in (1, -1):
+        kw = dict(dim=42, forward=fwd, flip_indices=flip if fwd < 0 else None)
+        g = batch.dop853_grid(MU, y0, 0.0, tf, m, **kw)
+        e = batch.dop853_final(MU, y0, 0.0, tf, variant="plain", **kw)
+        assert np.array_equal(g.states[:, -1].cpu().numpy(), e.y.cpu().numpy())
+        assert np.array_equal(g.n_accepted.cpu().numpy(), e.n_accepted.cpu().numpy())
+        shared = batch.dop853_grid(MU, y0, 0.0, 0.0, m, t_eval=t_eval, **kw)
+        sys = oracle.System("cr3bp42", mu=MU, fwd=fwd, flip=flip if fwd < 0 else None)
+        for i in some:
+            want = np.repeat(y0[i][None], m, 0) if tf[i] == 0.0 else \
+                oracle.compute_stm(MU, x[i], tf[i], steps=m, forward=fwd)[3]
+            assert np.array_equal(g.states[i].cpu().numpy(), want)
+            want = oracle.dop853(sys, y0[i], t_eval, rtol=1e-12, atol=1e-12, max_step=1e4)
+            assert np.array_equal(shared.states[i].cpu().numpy(), want[0])
+    cut = batch.dop853_grid(MU, y0, 0.0, tf, m, dim=42, max_steps=5)
+    end = batch.dop853_final(MU, y0, 0.0, tf, dim=42, max_steps=5, variant="plain")
+    assert np.array_equal(cut.status.cpu().numpy(), end.status.cpu().numpy())
+    assert np.array_equal(cut.states[:, -1].cpu().numpy(), end.y.cpu().numpy())
+
+
+@pytest.mark.parametrize("n", [4096, 4097])
+def test_open_variant_on_either_side_of_its_rule(gpu, n):
+    """dop853_final's 42-d default against the plain kernel, uneven spans with
+    zero and reversed ones among them."""
+    rng = np.random.default_rng(n)
+    y0 = W.with_identity_stm(W.planar_seeds(rng, n))
+    tf = rng.uniform(0.1, 1.0, n)
+    tf[5], tf[6] = 0.0, -0.5
+    a = batch.dop853_final(MU, y0, 0.0, tf, dim=42)
+    b = batch.dop853_final(MU, y0, 0.0, tf, dim=42, variant="plain")
+    for u, v in zip(vars(a).values(), vars(b).values()):
+        assert np.array_equal(u.cpu().numpy(), v.cpu().numpy())
