@@ -57,12 +57,17 @@ def _device() -> torch.device:
 
 
 def _vec(x, n: int, name: str) -> torch.Tensor:
-    """(n,) float64 device tensor from a scalar or array."""
+    """(n,) float64 device tensor from a scalar or array.  A host scalar is
+    written by a fill kernel: an upload of one value makes the host wait for
+    the stream."""
     dev = _device()
     if isinstance(x, torch.Tensor):
         t = x.to(device=dev, dtype=torch.float64)
     else:
-        t = torch.as_tensor(np.asarray(x, dtype=np.float64), device=dev)
+        a = np.asarray(x, dtype=np.float64)
+        if a.ndim == 0:
+            return torch.full((n,), float(a), dtype=torch.float64, device=dev)
+        t = torch.as_tensor(a, device=dev)
     if t.ndim == 0:
         t = t.expand(n)
     if t.shape != (n,):
@@ -386,7 +391,8 @@ def dop853_grid(mu, y0, t0, tf, m: int, *, dim: int = 6, t_eval=None, rtol: floa
     if t_eval is not None:
         te = _vec(t_eval, len(t_eval), "t_eval")
         m = te.shape[0]
-        t0, tf = float(te[0]), float(te[-1])
+        # the ends of host times are read on the host
+        t0, tf = float(t_eval[0]), float(t_eval[-1])
     mu_t, t0_t, tf_t = _vec(mu, n, "mu"), _vec(t0, n, "t0"), _vec(tf, n, "tf")
     out = torch.empty((n, int(m), dim), dtype=torch.float64, device=y.device)
     i32 = dict(dtype=torch.int32, device=y.device)

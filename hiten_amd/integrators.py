@@ -168,7 +168,8 @@ def _constant_solution(system, y0, t_vals):
 
 
 def _derivatives(system, mu, dim, fwd, flip, states):
-    """f(t, y) at every output state, evaluated by the GPU vector field."""
+    """f(t, y) at every output state (host rows, or rows still on the GPU),
+    evaluated by the GPU vector field."""
     d = batch.eval_rhs(mu, states, dim=dim).cpu().numpy()
     if fwd == -1:
         mask = batch.flip_mask(dim, flip)
@@ -302,11 +303,12 @@ class _DOP853(_AdaptiveStepRK):
             res = batch.dop853_final(mu, y0[None, :], t_vals[0], t_vals[-1], dim=dim, forward=fwd,
                                      flip_indices=flip, **step_kw)
             states = np.vstack([y0, res.y[0].cpu().numpy()])
+            derivs = _derivatives(system, mu, dim, fwd, flip, states)
         else:
             res = batch.dop853_grid(mu, y0[None, :], None, None, 0, dim=dim, t_eval=t_vals,
                                     forward=fwd, flip_indices=flip, **step_kw)
+            derivs = _derivatives(system, mu, dim, fwd, flip, res.states[0])
             states = res.states[0].cpu().numpy()
-        derivs = _derivatives(system, mu, dim, fwd, flip, states)
         return _Solution(times=t_vals.copy(), states=states, derivatives=derivs)
 
 

@@ -28,6 +28,7 @@ from dataclasses import dataclass, field
 from typing import List, Literal, Optional, Tuple
 
 import numpy as np
+import torch
 
 from .trajectory import Trajectory
 from . import batch
@@ -286,10 +287,13 @@ def compute_manifold(mu: float, orbit_state, period: float, *, stable: bool = Tr
     times = forward * np.linspace(0.0, tf, steps)
     # a NaN minimum compares false, as numpy's r1.min() < safe_r1 does
     kept = ~((r1 < safe_r1) | (r2 < safe_r2)) & ~(err > energy_tol)
-    host = states.cpu().numpy() if kept.any() else None
-    for i in np.nonzero(kept)[0]:
-        res.states_list.append(host[i].copy())
-        res.times_list.append(times.copy())
+    if kept.any():
+        # only the kept arcs come back, each a row of one host block
+        idx = np.nonzero(kept)[0]
+        if len(idx) < n:
+            states = states[torch.as_tensor(idx, device=states.device)]
+        res.states_list = list(states.contiguous().cpu().numpy())
+        res.times_list = [times.copy() for _ in idx]
     res.successes = int(kept.sum())
     res.seeds, res.kept = seeds, kept
     res.min_r1, res.min_r2, res.energy_err = r1, r2, err
