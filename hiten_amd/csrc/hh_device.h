@@ -122,16 +122,117 @@ __device__ __forceinline__ void pow_tab_fill(PowTab* t) {
     }
 }
 
-/* hh_pow on the tables at t (same bits as hh_pow) */
-__device__ __forceinline__ double pow_tab(const PowTab* t, double x, double y) {
-    return hh_pow_t(x, y, t->invc, t->log_hi, t->log_lo, t->exp_hi, t->exp_lo);
-}
-
 }  // namespace hh
 
 #include "hh_fast.h"
 
 namespace hh {
+
+/* hh_pow_t for a positive normal x and |y| <= 1/8, without its branches: the
+ * same operations in the same order, so the same bits.  The result lies in
+ * [2^-129, 2^129], so it neither over- nor underflows and one exact scaling
+ * replaces two.  Other x give an unused value.  The step controller lies on
+ * every trajectory's chain: without the branches one trajectory's attempt
+ * takes 3.56 instead of 3.74 us in a wave pair, 4.88 instead of 5.10 us in a
+ * wave, and 32,768 event searches 0.54 instead of 0.55 ms (lane groups).   */
+template <class Tab>
+__device__ __forceinline__ double pow_tab_normal(const Tab* pt, double x, double y) {
+    const int hi = __double2hiint(x);
+    const double kd = (double)((int)(((unsigned)hi >> 20) & 0x7ff) - 1023);
+    const int i = (hi >> 13) & 0x7f;
+    const double m = __hiloint2double((hi & 0x000fffff) | 0x3ff00000, __double2loint(x));
+    const double c = __hiloint2double(0x3ff00000 | (i << 13), 0);   /* 1 + i/128 */
+    const double dlt = m - c;
+    const double ic = pt->invc[i];
+    const double zh = dlt * ic;
+    const double zl = __builtin_fma(-zh, c, dlt) * ic;
+    double sq, sqe;
+    HH_TWO_PROD(zh, zh, sq, sqe);
+    double a_hi, a_lo;
+    HH_TWO_SUM(zh, -0.5 * sq, a_hi, a_lo);
+    const double w = zh;
+    const double tail = w * w * w * (1.0 / 3.0 - w * (0.25 - w * (0.2 - w * (1.0 / 6.0 - w * (
+        1.0 / 7.0 - w * (0.125 - w * (1.0 / 9.0 - w * 0.1)))))));
+    const double small = (-0.5 * sqe + (zl - zl * zh)) + tail;
+    double s1, e1, s2, e2;
+    HH_TWO_SUM(kd * HH_POW_LN2_HI, pt->log_hi[i], s1, e1);
+    HH_TWO_SUM(s1, a_hi, s2, e2);
+    const double l_lo = ((e1 + e2) + (kd * HH_POW_LN2_LO + pt->log_lo[i])) + (a_lo + small);
+    double l_hi, l_lo2;
+    HH_TWO_SUM(s2, l_lo, l_hi, l_lo2);
+    double t_hi, t_lo;
+    HH_TWO_PROD(y, l_hi, t_hi, t_lo);
+    t_lo = t_lo + y * l_lo2;
+    const double nd = (t_hi * HH_POW_INV_L128 + 6755399441055744.0) - 6755399441055744.0;
+    const int n = (int)nd;
+    const int j = n & 127;
+    const double r_hi = t_hi - nd * HH_POW_L128_HI;
+    const double r_lo = t_lo - nd * HH_POW_L128_LO;
+    double r, rr;
+    HH_TWO_SUM(r_hi, r_lo, r, rr);
+    const double q = r * r * (0.5 + r * (1.0 / 6.0 + r * (1.0 / 24.0 + r * (1.0 / 120.0 + r * (
+        1.0 / 720.0))))) + (rr + rr * r);
+    double e_hi, e_lo;
+    HH_TWO_SUM(1.0, r, e_hi, e_lo);
+    e_lo = e_lo + q;
+    const double xh = pt->exp_hi[j];
+    double p_hi, p_lo;
+    HH_TWO_PROD(xh, e_hi, p_hi, p_lo);
+    p_lo = p_lo + (xh * e_lo + pt->exp_lo[j] * e_hi);
+    return __builtin_ldexp(p_hi + p_lo, n >> 7);
+}
+
+/* the tables where they are defined, for the layouts without a copy of them */
+struct PowRef {
+    const double *invc, *log_hi, *log_lo, *exp_hi, *exp_lo;
+};
+__device__ __forceinline__ PowRef pow_ref() {
+    return PowRef{HH_POW_INVC, HH_POW_LOG_HI, HH_POW_LOG_LO, HH_POW_EXP_HI, HH_POW_EXP_LO};
+}
+template <class Tab>
+__device__ __forceinline__ double pow_any(const Tab* t, double x, double y) {
+    return hh_pow_t(x, y, t->invc, t->log_hi, t->log_lo, t->exp_hi, t->exp_lo);
+}
+
+/* a base pow_tab_normal takes, or one whose power is not used (err_prev = -1) */
+__device__ __forceinline__ bool pow_normal(double x) {
+    return (x >= 2.2250738585072014e-308 && x < __builtin_inf()) || x < 0.0;
+}
+
+/* pi_accept_factor and pi_reject_factor (below) from one power per lane: px
+ * and pe are the lane's base and exponent -- err^-beta, err_prev^alpha or
+ * err^(-1/8) -- and pick(v, i) the i-th power of the lane's trajectory.  With
+ * every base of the wave normal (err_prev = -1, a first step, is not used) the
+ * powers and the two factors are formed without branches.                 */
+template <class Tab, class Pick>
+__device__ __forceinline__ void step_factors_from(const Tab* pt, double err, double err_prev,
+                                                  double px, double pe, Pick pick, double& f_acc,
+                                                  double& f_rej) {
+    if (__builtin_expect(!__any(!pow_normal(px)), 1)) {
+        const double pw = pow_tab_normal(pt, px, pe);
+        const double pa = pick(pw, 1);
+        const double f = (0.9 * pick(pw, 0)) * (err_prev < 0.0 ? 1.0 : pa);
+        const double g = 0.9 * pick(pw, 2);
+        f_acc = __builtin_fmin(__builtin_fmax(f, 0.2), 10.0);
+        f_rej = __builtin_fmin(__builtin_fmax(g, 0.2), 10.0);
+        return;
+    }
+    const double pw = pow_any(pt, px, pe);
+    const double pb = pick(pw, 0), pa = pick(pw, 1), pr = pick(pw, 2);
+    double f;
+    if (err == 0.0) f = 10.0;
+    else if (err_prev < 0.0) f = 0.9 * pb;
+    else f = (0.9 * pb) * pa;
+    if (!(f == f)) f = 10.0;
+    if (f < 0.2) f = 0.2;
+    if (f > 10.0) f = 10.0;
+    f_acc = f;
+    double g = (err <= 0.0) ? 0.2 : 0.9 * pr;
+    if (!(g == g)) g = 0.2;
+    if (g < 0.2) g = 0.2;
+    if (g > 10.0) g = 10.0;
+    f_rej = g;
+}
 
 constexpr int DOP_S = 12;     /* stages of one DOP853 step                 */
 constexpr int DOP_K = 13;     /* stored stage derivatives (k[12] = f(y_high)) */
@@ -513,21 +614,29 @@ __device__ __forceinline__ void group_step_factors(int b, double err, double err
     const double err_exp = 1.0 / 8.0;
     const double px = (b == 1) ? err_prev : err;
     const double pe = (b == 0) ? -beta : ((b == 1) ? alpha : -err_exp);
-    const double pw = hh_pow(px, pe);
-    const double pb = group_get<0>(pw), pa = group_get<1>(pw), pr = group_get<2>(pw);
-    double f;
-    if (err == 0.0) f = 10.0;
-    else if (err_prev < 0.0) f = 0.9 * pb;
-    else f = (0.9 * pb) * pa;
-    if (!(f == f)) f = 10.0;
-    if (f < 0.2) f = 0.2;
-    if (f > 10.0) f = 10.0;
-    f_acc = f;
-    double g = (err <= 0.0) ? 0.2 : 0.9 * pr;
-    if (!(g == g)) g = 0.2;
-    if (g < 0.2) g = 0.2;
-    if (g > 10.0) g = 10.0;
-    f_rej = g;
+    const PowRef ref = pow_ref();
+    step_factors_from(&ref, err, err_prev, px, pe, [](double v, int i) {
+        return i == 0 ? group_get<0>(v) : (i == 1 ? group_get<1>(v) : group_get<2>(v));
+    }, f_acc, f_rej);
+}
+
+/* pi_accept_factor(err, err_prev) where err <= 1, else pi_reject_factor(err),
+ * of a trajectory per lane: two powers whatever the lanes of the wave decide,
+ * where the two factors formed in their branches take three (32,768 event
+ * searches 0.89 -> 0.78 ms, 131,072 end states 1.94 -> 1.82 ms)           */
+__device__ __forceinline__ double lane_step_factor(double err, double err_prev) {
+    const double beta = 1.0 / (8.0 + 1.0);
+    const double alpha = 0.4 * beta;
+    const double err_exp = 1.0 / 8.0;
+    const bool acc = err <= 1.0;
+    if (__builtin_expect(!__any(!pow_normal(err) || !pow_normal(err_prev)), 1)) {
+        const PowRef ref = pow_ref();
+        const double p1 = pow_tab_normal(&ref, err, acc ? -beta : -err_exp);
+        const double p2 = pow_tab_normal(&ref, err_prev, alpha);
+        const double f = (0.9 * p1) * (acc && !(err_prev < 0.0) ? p2 : 1.0);
+        return __builtin_fmin(__builtin_fmax(f, 0.2), 10.0);
+    }
+    return acc ? pi_accept_factor(err, err_prev) : pi_reject_factor(err);
 }
 
 /* rk.py:2443-2448 */

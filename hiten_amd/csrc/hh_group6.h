@@ -397,21 +397,9 @@ struct Lanes6 {
         const double err_exp = 1.0 / 8.0;
         const double px = (d == 1) ? err_prev : err;
         const double pe = (d == 0) ? -beta : ((d == 1) ? alpha : -err_exp);
-        const double pw = pow_tab(pt, px, pe);
-        const double pb = get<0>(pw), pa = get<1>(pw), pr = get<2>(pw);
-        double f;
-        if (err == 0.0) f = 10.0;
-        else if (err_prev < 0.0) f = 0.9 * pb;
-        else f = (0.9 * pb) * pa;
-        if (!(f == f)) f = 10.0;
-        if (f < 0.2) f = 0.2;
-        if (f > 10.0) f = 10.0;
-        f_acc = f;
-        double g = (err <= 0.0) ? 0.2 : 0.9 * pr;
-        if (!(g == g)) g = 0.2;
-        if (g < 0.2) g = 0.2;
-        if (g > 10.0) g = 10.0;
-        f_rej = g;
+        step_factors_from(pt, err, err_prev, px, pe, [this](double v, int i) {
+            return i == 0 ? get<0>(v) : (i == 1 ? get<1>(v) : get<2>(v));
+        }, f_acc, f_rej);
     }
 
     /* the three extension stages and the seven interpolant rows of this

@@ -202,10 +202,11 @@ __device__ __forceinline__ void traj_iterate(const P& p, Traj<P>& s, const StepP
         o.stop(s.y);
         return;
     }
-    /* Lane42: both factors from one pow per lane of the group, formed
-     * before the group-uniform branch; Lane6: the factor its branch needs */
-    double f_acc = 0.0, f_rej = 0.0;
+    /* formed before the branch: Lane42 both factors from one pow per lane of
+     * the group, Lane6 the one its branch needs from two                  */
+    double f_acc, f_rej;
     if constexpr (P::N == 42) group_step_factors(p.blk, err, s.err_prev, f_acc, f_rej);
+    else f_acc = f_rej = lane_step_factor(err, s.err_prev);
     if (err <= 1.0) {
         const double t_new = s.t + h;
         const bool last = !((t_new - s.tf) * 1.0 < 0.0);
@@ -217,12 +218,10 @@ __device__ __forceinline__ void traj_iterate(const P& p, Traj<P>& s, const StepP
             s.y[d] = yh[d];
             s.k[0][d] = s.k[DOP_S][d];
         }
-        if constexpr (P::N != 42) f_acc = pi_accept_factor(err, s.err_prev);
         s.h = h * f_acc;
         s.err_prev = err;
         s.nacc += 1;
     } else {
-        if constexpr (P::N != 42) f_rej = pi_reject_factor(err);
         s.h = clamp_step(h * f_rej, sp.max_step, sp.min_step);
         s.nrej += 1;
     }
@@ -736,6 +735,7 @@ __global__ __launch_bounds__(256) void k_dop853_event6(
             st = ST_NONFINITE;
             break;
         }
+        const double factor = lane_step_factor(err, err_prev);
         if (err <= 1.0) {
             const double t_new = t + h;
             const double gn = pick6(yh, ev.index) - ev.offset;
@@ -768,10 +768,10 @@ __global__ __launch_bounds__(256) void k_dop853_event6(
                 k[0][d] = k[DOP_S][d];
             }
             gp = gn;
-            h = h * pi_accept_factor(err, err_prev);
+            h = h * factor;
             err_prev = err;
         } else {
-            h = clamp_step(h * pi_reject_factor(err), sp.max_step, sp.min_step);
+            h = clamp_step(h * factor, sp.max_step, sp.min_step);
             nr += 1;
         }
     }

@@ -21,11 +21,13 @@
  * general forms, from the flags both waves write beside the sums.
  *
  * Bound by the longer of the two instruction streams and the LDS round trip
- * and barrier of every stage.  One trajectory alone: 3.95 us an attempt (5.83
+ * and barrier of every stage.  One trajectory alone: 3.56 us an attempt (5.83
  * us with twelve quotients read back by readlane, IEEE divisions and both
- * roles in one stream; 4.22 us before each role had a stream of its own),
- * 5.10 us in the one-wave form (6.75 us).  262,144 uneven trajectories on the
- * persistent kernel, whose heaviest ones end in this form: 94 -> 62 ms.
+ * roles in one stream; 4.22 us before each role had a stream of its own, 3.94
+ * us before the state row hid the record's stores, 3.74 us before the step
+ * controller lost its branches), 4.88 us in the one-wave form (6.75 us).
+ * 262,144 uneven trajectories on the persistent kernel, whose heaviest ones
+ * end in this form: 94 -> 59 ms.
  */
 #ifndef HH_PAIR_H
 #define HH_PAIR_H
@@ -83,8 +85,12 @@ struct Pair42 : Var42 {
             const double q = quotient<FAST>(v, c, w, u);
             lds->rec[BUF].q[lane] = q;
             lds->rec[BUF].u[lane] = u;
+            /* the state row while the stores are on their way: the barrier
+             * waits for them                                               */
+            double o = xor_sign(state_row<FAST>(v, q, w), sign);
+            asm volatile("" : "+v"(o));
             __syncthreads();
-            return xor_sign(state_row<FAST>(v, q, w), sign);
+            return o;
         } else {
             __syncthreads();
             return xor_sign(column_row<FAST>(v, mine[BUF]), sign);

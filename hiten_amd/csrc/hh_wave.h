@@ -281,21 +281,8 @@ struct Var42 {
         const double err_exp = 1.0 / 8.0;
         const double px = (lane == 1) ? err_prev : err;
         const double pe = (lane == 0) ? -beta : ((lane == 1) ? alpha : -err_exp);
-        const double pw = pow_tab(pt, px, pe);
-        const double pb = rlane(pw, 0), pa = rlane(pw, 1), pr = rlane(pw, 2);
-        double f;
-        if (err == 0.0) f = 10.0;
-        else if (err_prev < 0.0) f = 0.9 * pb;
-        else f = (0.9 * pb) * pa;
-        if (!(f == f)) f = 10.0;
-        if (f < 0.2) f = 0.2;
-        if (f > 10.0) f = 10.0;
-        f_acc = f;
-        double g = (err <= 0.0) ? 0.2 : 0.9 * pr;
-        if (!(g == g)) g = 0.2;
-        if (g < 0.2) g = 0.2;
-        if (g > 10.0) g = 10.0;
-        f_rej = g;
+        step_factors_from(pt, err, err_prev, px, pe,
+                          [](double v, int i) { return rlane(v, i); }, f_acc, f_rej);
     }
 };
 

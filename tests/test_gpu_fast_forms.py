@@ -175,3 +175,24 @@ def test_open_variant_on_either_side_of_its_rule(gpu, n):
     b = batch.dop853_final(MU, y0, 0.0, tf, dim=42, variant="plain")
     for u, v in zip(vars(a).values(), vars(b).values()):
         assert np.array_equal(u.cpu().numpy(), v.cpu().numpy())
+
+
+@pytest.mark.parametrize("dim,variant", [(6, "plain"), (6, "wide"), (42, "plain"), (42, "wide"),
+                                         (42, "pair"), (42, "persistent")])
+@pytest.mark.parametrize("atol", [1e140, 1e152, 1e158, 1e200, 1e292])
+def test_step_control_with_vanishing_errors(gpu, oracle, dim, variant, atol):
+    """Error norms that underflow, or are exactly zero, as the controller's
+    bases err and err_prev; large steps, the end's short ones."""
+    n = 20
+    rng = np.random.default_rng(4)
+    x = W.planar_seeds(rng, n)
+    y0 = x if dim == 6 else W.with_identity_stm(x)
+    tf = rng.uniform(1e-4, 0.2, n)
+    r = batch.dop853_final(MU, y0, 0.0, tf, dim=dim, atol=atol, variant=variant, max_step=0.01,
+                           max_steps=300)
+    want, na, nr, st = oracle.batch_dop853_final(np.full(n, MU), y0, np.zeros(n), tf, atol=atol,
+                                                 max_step=0.01, max_steps=300)
+    assert np.array_equal(r.y.cpu().numpy(), want)
+    assert np.array_equal(r.n_accepted.cpu().numpy(), na)
+    assert np.array_equal(r.n_rejected.cpu().numpy(), nr)
+    assert np.array_equal(r.status.cpu().numpy(), st)
