@@ -529,13 +529,18 @@ __device__ __forceinline__ void syn_candidate(const SynArgs& a, const SynSeg& g,
 }
 
 /* The multi-pass form.  Pass 1 scans every part of SYN_PART segments of
- * every trajectory with a wave of its own and appends its candidates, with
- * their places in segment order, to compact lists; pass 2 refines the
+ * every trajectory with a wave of its own -- a division-free test finds the
+ * few segments that may hold a candidate, those are walked one per lane -- and
+ * appends its candidates, with their places in segment order, to compact
+ * lists; pass 2 refines the
  * listed candidates, one per lane of a dense grid; pass 3 deduplicates
  * each trajectory's refined candidates in order.  Candidates come from the
  * same segment values, walk and refinement as in syn_detect_wave, so the
  * hits are the same bits.                                                 */
-constexpr int SYN_PART = 512;     /* segments per part (8 chunks of 64)        */
+constexpr int SYN_CHUNK = 61;     /* segments a wave tests at once: 64 samples,
+                                     less one before and two after            */
+constexpr int SYN_BATCH = 4;      /* chunks in flight                          */
+constexpr int SYN_PART = 8 * SYN_CHUNK;   /* segments per part                 */
 constexpr int SYN_CAP = 32;       /* refined candidates recorded per part      */
 constexpr int SYN_REC = 7;        /* doubles of a refined candidate: t, x[6]   */
 constexpr int SYN_LISTS = 8;      /* candidate lists (part index % SYN_LISTS),
@@ -555,10 +560,44 @@ struct SynWs {
                                      candidates, component-major per part      */
 };
 
+/* lane i takes lane i + 1 (i - 1) of the wave; 0 past its ends */
+__device__ __forceinline__ double wave_next(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x130, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x130, 0xF, 0xF, true);
+    return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double wave_prev(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x138, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x138, 0xF, 0xF, true);
+    return __hiloint2double(hi, lo);
+}
+
+/* The segments (bit l: the one that starts at lane l's sample, lanes 1 ..
+ * SYN_CHUNK) that may hold a candidate, from the plane value g and time t of
+ * one sample per lane.  A segment is left out when its ends are on one side of
+ * the plane, sample k is not on it, and no interpolant value can reach it: the
+ * Hermite cubic differs from a convex combination of the ends by at most 4/27
+ * dt (|d0| + |d1|) (syn_no_sign_change), where dt |d0| <= |g(k+1) - g(k-1)|
+ * and dt |d1| <= |g(k+2) - g(k)| as long as the four times do not decrease.
+ * With D(k) = |g(k+1) - g(k)| these are at most D(k-1) + D(k) and D(k) +
+ * D(k+1), no division needed; 0.15 > 4/27 and 1e-8 |g| leave more room than the
+ * rounding of the evaluated values takes.  NaN fails the test.            */
+__device__ __forceinline__ unsigned long long syn_suspects(const SynArgs& a, int N, int j, int lane,
+                                                           double g, double t) {
+    const bool pair = j >= 0 && j + 1 < N;
+    const double D = pair ? __builtin_fabs(wave_next(g) - g) : 0.0;
+    const unsigned long long rising = __ballot(!pair || t <= wave_next(t));
+    const double A = __builtin_fabs(g);
+    const bool clear = (A - D > 0.15 * ((D + D) + (wave_prev(D) + wave_next(D))) + 1e-8 * A) &&
+                       A >= a.tol_on;
+    return __ballot(!clear) | ~(rising & (rising << 1) & (rising >> 1));
+}
+
 /* Pass 1 for part p of trajectory i (one wave); `seg` is the wave's LDS
- * list of candidates (SYN_CAP entries).                                   */
+ * list of candidates (SYN_CAP entries), `sus` its list of segments that may
+ * hold one (SYN_PART entries).                                            */
 __device__ __forceinline__ void syn_scan_part(SynArgs a, const SynWs& w, int i, int p,
-                                              int lane, int4* seg) {
+                                              int lane, int4* seg, short* sus) {
     SynTraj tr;
     tr.a = &a;
     tr.base = (size_t)i * a.m;
@@ -568,42 +607,57 @@ __device__ __forceinline__ void syn_scan_part(SynArgs a, const SynWs& w, int i, 
     const int s0 = p * SYN_PART;
     const int s1 = min(s0 + SYN_PART, nseg);
     const int unit = i * w.parts + p;
-    int found = 0;        /* candidates so far */
-    auto extra = [&](int k0) {
-        return (lane == 0) ? k0 - 1 : ((lane == 62) ? k0 + 64 : ((lane == 63) ? k0 + 65 : -1));
-    };
-    double xo[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}, to = 0.0;
-    double xe[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}, te = 0.0;
-    if (s0 < s1) {
-        if (s0 + lane < tr.N) tr.load(s0 + lane, xo, to);
-        const int jx = extra(s0);
-        if (jx >= 0 && jx < tr.N) tr.load(jx, xe, te);
-    }
-    for (int k0 = s0; k0 < s1; k0 += 64) {
-        const int k = k0 + lane;
-        const double gj = (k < tr.N) ? tr.G(xo) : 0.0;
-        const double tj = (k < tr.N) ? to : 0.0;
-        const int jx = extra(k0);
-        const bool ex = jx >= 0 && jx < tr.N;
-        const double gx = ex ? tr.G(xe) : 0.0;
-        const double tx = ex ? te : 0.0;
-        if (k0 + 64 < s1) {
-            if (k + 64 < tr.N) tr.load(k + 64, xo, to);
-            const int jn = extra(k0 + 64);
-            if (jn >= 0 && jn < tr.N) tr.load(jn, xe, te);
+    /* the samples, SYN_BATCH chunks in flight at once: lane l holds sample k0 -
+     * 1 + l of a chunk of SYN_CHUNK segments k0 .., so that each segment finds
+     * its neighbours' values in the wave                                    */
+    int nsus = 0;
+    for (int b0 = s0; b0 < s1; b0 += SYN_BATCH * SYN_CHUNK) {
+        double x[SYN_BATCH][6], t[SYN_BATCH];
+#pragma unroll
+        for (int c = 0; c < SYN_BATCH; ++c) {
+            const int j = b0 + c * SYN_CHUNK - 1 + lane;
+            t[c] = 0.0;
+#pragma unroll
+            for (int d = 0; d < 6; ++d) x[c][d] = 0.0;
+            if (j >= 0 && j < tr.N && j <= s1 + 1) tr.load(j, x[c], t[c]);
         }
-        const double g_up1 = __shfl(gj, (lane + 1) & 63), t_up1 = __shfl(tj, (lane + 1) & 63);
-        const double g_up2 = __shfl(gj, (lane + 2) & 63), t_up2 = __shfl(tj, (lane + 2) & 63);
-        const double g_dn1 = __shfl(gj, (lane + 63) & 63), t_dn1 = __shfl(tj, (lane + 63) & 63);
-        const double g_x62 = __shfl(gx, 62), t_x62 = __shfl(tx, 62);
-        const double g_x63 = __shfl(gx, 63), t_x63 = __shfl(tx, 63);
-        const double gk1 = (lane < 63) ? g_up1 : g_x62, tk1 = (lane < 63) ? t_up1 : t_x62;
-        const double gk2 = (lane < 62) ? g_up2 : ((lane == 62) ? g_x62 : g_x63);
-        const double tk2 = (lane < 62) ? t_up2 : ((lane == 62) ? t_x62 : t_x63);
-        const double gkm1 = (lane > 0) ? g_dn1 : gx, tkm1 = (lane > 0) ? t_dn1 : tx;
-        int cnt = 0;
-        if (k < s1) {
-            const SynSeg g = syn_segment(a, tr.N, k, gkm1, gj, gk1, gk2, tkm1, tj, tk1, tk2);
+#pragma unroll
+        for (int c = 0; c < SYN_BATCH; ++c) {
+            const int k0 = b0 + c * SYN_CHUNK;
+            const int j = k0 - 1 + lane;
+            unsigned long long m = syn_suspects(a, tr.N, j, lane, tr.G(x[c]), t[c]);
+            /* lanes 1 .. SYN_CHUNK start this chunk's segments */
+            const int n = min(SYN_CHUNK, s1 - k0);
+            if (n <= 0) break;
+            m &= (((1ULL << n) - 1ULL) << 1);
+            if (m >> lane & 1ULL)
+                sus[nsus + __popcll(m & ((1ULL << lane) - 1ULL))] = (short)(j - s0);
+            nsus += __popcll(m);
+        }
+    }
+    /* the segments that may hold candidates, one per lane: their candidates
+     * counted as syn_detect_wave counts them                                */
+    int found = 0;        /* candidates so far */
+    __builtin_amdgcn_wave_barrier();
+    for (int q0 = 0; q0 < nsus; q0 += 64) {
+        int cnt = 0, k = 0;
+        if (q0 + lane < nsus) {
+            k = s0 + sus[q0 + lane];
+            const bool m1 = k >= 1, p2 = k + 2 < tr.N;
+            double xv[6], gkm1 = 0.0, gk2 = 0.0, tm1 = 0.0, t0, t1, t2 = 0.0;
+            if (m1) {
+                tr.load(k - 1, xv, tm1);
+                gkm1 = tr.G(xv);
+            }
+            if (p2) {
+                tr.load(k + 2, xv, t2);
+                gk2 = tr.G(xv);
+            }
+            tr.load(k, xv, t0);
+            const double gk = tr.G(xv);
+            tr.load(k + 1, xv, t1);
+            const double gk1 = tr.G(xv);
+            const SynSeg g = syn_segment(a, tr.N, k, gkm1, gk, gk1, gk2, tm1, t0, t1, t2);
             syn_walk(a, g, -1, &cnt);
         }
         if (__ballot(cnt > 0)) {
@@ -632,17 +686,21 @@ __device__ __forceinline__ void syn_scan_part(SynArgs a, const SynWs& w, int i, 
     if (lane < found) w.list[(size_t)li * w.cap_list + base + lane] = seg[lane];
 }
 
-/* Four waves per SIMD fit without spills; three, with a second chunk in
- * flight per wave, measured slower (288 against 247 us on 4,096 x 4,713
- * samples).                                                               */
+/* Bound by HBM: 4,096 x 4,713 samples (928 MB) in 179 us, 5.2 TB/s, of the 6.2
+ * TB/s a plain read reaches; 225 us (4.1 TB/s) while every segment's slopes
+ * were divided out and its walk begun, about 250 instructions a chunk instead
+ * of 60, with one chunk in flight.  Four chunks at four waves a SIMD: two
+ * chunks 27 us a call slower, five or six waves no faster.                */
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void k_synodic_scan(SynArgs a, SynWs w) {
     __shared__ int4 seg[BLOCK / 64][SYN_CAP];
+    __shared__ short sus[BLOCK / 64][SYN_PART];
     const long long wave = ((long long)blockIdx.x * BLOCK + threadIdx.x) >> 6;
     if (wave >= (long long)a.n * w.parts) return;
-    syn_scan_part(a, w, (int)(wave / w.parts), (int)(wave % w.parts), threadIdx.x & 63,
-                  seg[threadIdx.x >> 6]);
+    const int wid = threadIdx.x >> 6;
+    syn_scan_part(a, w, (int)(wave / w.parts), (int)(wave % w.parts), threadIdx.x & 63, seg[wid],
+                  sus[wid]);
 }
 
 /* Pass 2: every listed candidate in a lane of its own (a grid-stride loop

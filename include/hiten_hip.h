@@ -280,7 +280,7 @@ int hh_synodic_detect(int n, int m, const double* times, int per_traj_times,
                       double dedup_point_tol, int max_hits, int newton_max_iter, int cap,
                       int* count, double* hit_t, double* hit_x, double* hit_p, void* stream);
 
-/* hh_synodic_detect in passes: every part of 512 segments of every
+/* hh_synodic_detect in passes: every part of 488 segments of every
  * trajectory is scanned by a wave of its own, which lists the segments
  * holding candidates; the listed segments are refined one per lane; then
  * one wave per trajectory deduplicates the refined candidates in segment
