@@ -29,7 +29,8 @@
  * Measured against the form before (components in lanes 0..5, LDS swizzles,
  * IEEE divisions and branches): 1,024 x 2,000 RK8 steps 7.29 -> 3.81 ms (153
  * ns a stage, about 75 instructions of a wave alone on its SIMD), 500
- * manifold arcs 5.31 -> 3.36 ms, 32,768 event searches 0.72 -> 0.59 ms.
+ * manifold arcs 5.31 -> 3.36 ms (1.28 with group6_points), 32,768 event
+ * searches 0.72 -> 0.59 ms.
  */
 #ifndef HH_GROUP6_H
 #define HH_GROUP6_H

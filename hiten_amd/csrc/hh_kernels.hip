@@ -549,6 +549,72 @@ __device__ __forceinline__ bool cancelled(const int* flag) {
     return false;
 }
 
+/* The points from q on that a step from t to t_new covers (GridOut).  Returns
+ * the first point left over.
+ *
+ * A row of 16 lanes takes one point a lane: time, abscissa and six components
+ * of 16 points are formed at once, each component from rows that are broadcast
+ * over the group, in about 190 instructions, where one point after the other
+ * waits for a division and the serial interpolant each time.  The row's
+ * interpolant, points and stages together need 204 registers, and 1,024 waves
+ * are all there are (ROW6_MAX): two waves to a SIMD cost nothing, a limit of
+ * 128 registers (74 spilled) does.  500 arcs of 4,713 points 3.34 -> 1.28 ms;
+ * at 200 points 0.99 and 0.95 ms.
+ *
+ * In a group of 8 lanes a broadcast is four moves and the SIMDs are shared:
+ * 8,192 arcs take 2.41 ms point by point and 2.16 ms that way at 1,000 points,
+ * but 1.56 and 1.69 ms at 100, so they stay with one point at a time.        */
+template <class P, class TQ>
+__device__ __forceinline__ int group6_points(const P& p, const double (&row)[DOP_P], double y,
+                                             double t, double t_new, double hs, bool last, int q,
+                                             int m, const TQ& tq, double* gout) {
+    if constexpr (P::LANES == 8) {
+        for (; q < m; ++q) {
+            const double t_q = tq(q);
+            if (!(last || t_q < t_new)) break;
+            const double v = dense_from_rows(row, y, (t_q - t) / hs);
+            if (p.act) gout[(size_t)q * 6 + p.d] = v;
+        }
+        return q;
+    }
+    const int l = p.lane & (P::LANES - 1);
+    const int first = p.lane & 63 & ~(P::LANES - 1);
+    while (q < m) {
+        const int i = q + l;
+        const double ti = tq(i < m ? i : m - 1);
+        const double x = (ti - t) / hs;
+        const bool in = i < m && (last || ti < t_new);
+        /* the points up to the first one this step does not cover */
+        const unsigned no = (unsigned)(~__ballot(in) >> first) & ((1u << P::LANES) - 1u);
+        const int cnt = no ? __ffs((int)no) - 1 : P::LANES;
+        const double omx = 1.0 - x;
+        double v[6];
+        auto component = [&](auto kc) {
+            constexpr int K = decltype(kc)::value;
+            double a = 0.0;   /* dense_from_rows */
+#pragma unroll
+            for (int r = DOP_P - 1; r >= 0; --r) {
+                a = a + p.template get<K>(row[r]);
+                a = a * (((DOP_P - 1 - r) % 2 == 0) ? x : omx);
+            }
+            v[K] = a + p.template get<K>(y);
+        };
+        component(std::integral_constant<int, 0>());
+        component(std::integral_constant<int, 1>());
+        component(std::integral_constant<int, 2>());
+        component(std::integral_constant<int, 3>());
+        component(std::integral_constant<int, 4>());
+        component(std::integral_constant<int, 5>());
+        if (l < cnt) {
+#pragma unroll
+            for (int c = 0; c < 6; ++c) gout[(size_t)i * 6 + c] = v[c];
+        }
+        q += cnt;
+        if (cnt < P::LANES) break;
+    }
+    return q;
+}
+
 /* One trajectory of k_dop853_run6 in a lane group (Group6 or Row6):
  * traj_init / traj_iterate and the FinalOut / GridOut policies, statement for
  * statement, with each lane holding its component: the grid form writes this lane's component of every output
@@ -577,6 +643,7 @@ __device__ __forceinline__ void group6_run(const P& p, double y, double t0, doub
         if (p.act) gout[(size_t)q * 6 + d] = v;
     };
     int q = 0;
+    double t_next = GRID ? tq(0) : 0.0;   /* time of point q */
     yfin = y;   /* FinalOut */
     double t = t0, h, err_prev = -1.0;
     int na = 0, nr = 0, st = ST_OK;
@@ -618,17 +685,14 @@ __device__ __forceinline__ void group6_run(const P& p, double y, double t0, doub
             const bool last = !((t_new - tf) * 1.0 < 0.0);
             const double hs = t_new - t;
             if constexpr (GRID) {
-                if (q < m && (last || tq(q) < t_new)) {
+                if (q < m && (last || t_next < t_new)) {
                     if (hs == 0.0) {
                         for (; q < m; ++q) put(q, y);
                     } else {
                         double row[DOP_P];
                         p.dense_rows(y, yh, k, hs, row);
-                        for (; q < m; ++q) {
-                            const double t_q = tq(q);
-                            if (!(last || t_q < t_new)) break;
-                            put(q, dense_from_rows(row, y, (t_q - t) / hs));
-                        }
+                        q = group6_points(p, row, y, t, t_new, hs, last, q, m, tq, gout);
+                        t_next = tq(q < m ? q : m - 1);
                     }
                 }
             } else {
@@ -660,7 +724,7 @@ __device__ __forceinline__ void group6_run(const P& p, double y, double t0, doub
 }
 
 template <class P, bool GRID>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GRID && P::LANES == 16 ? 2 : 4)))
 void k_dop853_run6_group(
     int n, const double* __restrict__ mu, const double* __restrict__ t0a,
     const double* __restrict__ tfa, StepParams sp, int fwd, unsigned long long flip,

@@ -196,3 +196,30 @@ def test_step_control_with_vanishing_errors(gpu, oracle, dim, variant, atol):
     assert np.array_equal(r.n_accepted.cpu().numpy(), na)
     assert np.array_equal(r.n_rejected.cpu().numpy(), nr)
     assert np.array_equal(r.status.cpu().numpy(), st)
+
+
+@pytest.mark.parametrize("n", [1, 6, 4097])
+@pytest.mark.parametrize("m", [2, 15, 17, 129, 1500])
+def test_grid_points_a_lane_each(gpu, n, m):
+    """6-d grids of lane groups (up to 4,096 trajectories sixteen points at
+    once) against one trajectory per lane: none, fewer and more points in a
+    step than a group has lanes, output times that repeat or go back, a span of
+    zero, an attempt limit, a step that covers points only at its end."""
+    rng = np.random.default_rng(100 * n + m)
+    y = W.planar_seeds(rng, n)
+    y[:, 1:3] = rng.uniform(-0.02, 0.02, (n, 2))
+    tf = rng.uniform(0.2, 1.5, n)
+    tf[n // 2] = 0.0 if n > 1 else tf[0]
+    t_eval = np.sort(rng.uniform(0.0, 0.7, m))
+    t_eval[0] = 0.0
+    again = t_eval.copy()
+    again[m // 2:m // 2 + 3] = again[m // 2]
+    back = t_eval.copy()
+    back[m // 3:m // 3 + 2] = back[m // 3:m // 3 + 2][::-1]
+    for fwd in (1, -1):
+        for kw in (dict(), dict(max_steps=5), dict(max_step=0.05, max_steps=9), dict(t_eval=t_eval),
+                   dict(t_eval=again), dict(t_eval=back)):
+            a, b = (batch.dop853_grid(MU, y, 0.0, tf if "t_eval" not in kw else 0.0, m, variant=v,
+                                      forward=fwd, **kw) for v in ("wide", "plain"))
+            for u, v in zip(vars(a).values(), vars(b).values()):
+                assert np.array_equal(u.cpu().numpy(), v.cpu().numpy())
