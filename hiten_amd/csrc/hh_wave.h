@@ -49,6 +49,10 @@ struct StageRec {
     double q[64], u[64];
 };
 
+/* Keeps the compiler to the order in which LDS accesses are written.  The LDS
+ * carries out one wave's accesses in the order they are issued.            */
+__device__ __forceinline__ void lds_order() { asm volatile("" ::: "memory"); }
+
 /* Lane layout, constants and the two halves of the field */
 struct Var42 {
     double mu, mu2;
@@ -177,27 +181,37 @@ struct Var42 {
         return (act && st) ? o : 0.0;
     }
 
-    /* derivative of this lane's column entry: row d of F @ Phi[:, j]
-     * (rtbp.py:124-141, column_rhs); r: the stage's record in velocity lanes,
-     * zeros in the others                                                   */
-    template <bool FAST>
-    __device__ __forceinline__ double column_row(double v, const StageRec& r) const {
+    /* What a column's lane reads of a stage's record */
+    struct Entries {
+        double Q6, Q7, Q8, Q9, Q10, Q11, y, z, pa, pb;
+    };
+    template <class R>
+    __device__ __forceinline__ Entries entries(const R& r) const {
         const int row = vel ? (l & 3) : 0;
-        const double pv = vel_entry(v);
+        return {r.q[8], r.q[10], r.q[7], r.q[15], r.q[9], r.q[11], r.u[5], r.u[6],
+                r.u[4 + row], r.u[12 + row]};   /* xm, y, z and xr, y, z */
+    }
+
+    /* derivative of this lane's column entry: row d of F @ Phi[:, j]
+     * (rtbp.py:124-141, column_rhs); r: from the stage's record in velocity
+     * lanes, zeros in the others                                              */
+    template <bool FAST>
+    __device__ __forceinline__ double column_row(double v, Entries r) const {
+        double pv = vel_entry(v);
         const double t = dpp_into<DPP_SHR4, BANKS_VEL>(v, v);
-        const double p0 = quad_get<0x00>(t), p1 = quad_get<0x55>(t), p2 = quad_get<0xAA>(t);
-        const double Q6 = r.q[8], Q7 = r.q[10], Q8 = r.q[7], Q9 = r.q[15];
-        const double Q10 = r.q[9], Q11 = r.q[11];
-        const double y = r.u[5], z = r.u[6];
-        const double pa = r.u[4 + row], pb = r.u[12 + row];   /* xm, y, z and xr, y, z */
-        const double a53 = Q6 * 3.0;
-        const double b53 = Q7 * 3.0;
-        const double c3 = Q8 + Q9;
-        const double gx = Q10 + Q11;
-        const double dd = ((diag + a53 * (pa * pa)) + b53 * (pb * pb)) - c3;
-        const double uxy = (3.0 * y) * gx;
-        const double uxz = (3.0 * z) * gx;
-        const double uyz = ((3.0 * y) * z) * (Q6 + Q7);
+        double p0 = quad_get<0x00>(t), p1 = quad_get<0x55>(t), p2 = quad_get<0xAA>(t);
+        asm volatile(""
+                     : "+v"(r.Q6), "+v"(r.Q7), "+v"(r.Q8), "+v"(r.Q9), "+v"(r.Q10), "+v"(r.Q11),
+                       "+v"(r.y), "+v"(r.z), "+v"(r.pa), "+v"(r.pb), "+v"(pv), "+v"(p0),
+                       "+v"(p1), "+v"(p2));
+        const double a53 = r.Q6 * 3.0;
+        const double b53 = r.Q7 * 3.0;
+        const double c3 = r.Q8 + r.Q9;
+        const double gx = r.Q10 + r.Q11;
+        const double dd = ((diag + a53 * (r.pa * r.pa)) + b53 * (r.pb * r.pb)) - c3;
+        const double uxy = (3.0 * r.y) * gx;
+        const double uxz = (3.0 * r.z) * gx;
+        const double uyz = ((3.0 * r.y) * r.z) * (r.Q6 + r.Q7);
         const double cA = (l == 4) ? dd : ((l == 5) ? uxy : uxz);
         const double cB = (l == 4) ? uxy : ((l == 5) ? dd : uyz);
         const double cC = (l == 4) ? uxz : ((l == 5) ? uyz : dd);
@@ -287,7 +301,11 @@ struct Var42 {
 };
 
 /* dop853_attempt's stages and solution, one component per lane; W supplies
- * the right-hand side of stage i (rhs_form<FAST, i % 2>)                   */
+ * the right-hand side; its last argument numbers those of an integration
+ * between two norms: 0..11 an attempt's, 12..14 the extension stages',
+ * RHS_START the start's                                                     */
+constexpr int RHS_START = 15;
+
 template <bool FAST, class W>
 __device__ __forceinline__ double dop853_stages(const W& w, double y, double (&k)[DOP_K], double h,
                                                 FastChk& c) {
@@ -299,14 +317,13 @@ __device__ __forceinline__ double dop853_stages(const W& w, double y, double (&k
 #pragma unroll
         for (int j = 0; j < i; ++j)
             if (HH_DOP_A[i][j] != 0.0) ys = ys + ha.at(n++) * k[j];
-        k[i] = (i % 2 == 0) ? w.template rhs_form<FAST, 0>(ys, c)
-                            : w.template rhs_form<FAST, 1>(ys, c);
+        k[i] = w.template rhs_form<FAST>(ys, c, i - 1);
     }
     double yh = y;
 #pragma unroll
     for (int j = 0; j < DOP_S; ++j)
         if (HH_DOP_B[j] != 0.0) yh = yh + ha.at(n++) * k[j];
-    k[DOP_S] = w.template rhs_form<FAST, 0>(yh, c);
+    k[DOP_S] = w.template rhs_form<FAST>(yh, c, DOP_S - 1);
     return yh;
 }
 
@@ -325,10 +342,7 @@ __device__ __forceinline__ void dop853_rows(const W& w, double y_old, double y_n
             const double a = HH_DOP_A[sr][r];
             if (a != 0.0) acc = acc + a * (r < DOP_K ? k[r] : kx[r - DOP_K]);
         }
-        const double ys = y_old + hs * acc;
-        kx[sr - DOP_K] = sr == DOP_K       ? w.template rhs<1>(ys)
-                         : sr == DOP_K + 1 ? w.template rhs<0>(ys)
-                                           : w.template rhs<2>(ys);
+        kx[sr - DOP_K] = w.rhs(y_old + hs * acc, sr - 1);
     }
     const double dy = y_new - y_old;
     row[0] = dy;
@@ -373,8 +387,8 @@ struct Wave42 : Var42 {
 
     /* derivative of this lane's component; v = this lane's component of the
      * stage state (idle() in lanes without one)                             */
-    template <bool FAST, int>
-    __device__ __forceinline__ double rhs_form(double v, FastChk& c) const {
+    template <bool FAST>
+    __device__ __forceinline__ double rhs_form(double v, FastChk& c, int = 0) const {
         double w, u;
         const double q = quotient<FAST>(v, c, w, u);
         rec->q[lane] = q;
@@ -383,8 +397,10 @@ struct Wave42 : Var42 {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const Entries e = entries(*mine);
+        lds_order();
         const double os = state_row<FAST>(v, q, w);
-        const double oc = column_row<FAST>(v, *mine);
+        const double oc = column_row<FAST>(v, e);
         __builtin_amdgcn_wave_barrier();
         return xor_sign(st ? os : oc, sign);
     }
@@ -394,13 +410,12 @@ struct Wave42 : Var42 {
         return st && c.outside();
     }
 
-    template <int BUF = 0>
-    __device__ __forceinline__ double rhs(double v) const {
+    __device__ __forceinline__ double rhs(double v, int = 0) const {
         FastChk c;
         c.num(mu);
         c.num(mu2);
-        const double o = rhs_form<true, BUF>(v, c);
-        if (__builtin_expect(__any(left_range(c)), 0)) return rhs_form<false, BUF>(v, c);
+        const double o = rhs_form<true>(v, c);
+        if (__builtin_expect(__any(left_range(c)), 0)) return rhs_form<false>(v, c);
         return o;
     }
 
