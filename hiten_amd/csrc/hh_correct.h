@@ -526,7 +526,7 @@ __device__ __forceinline__ void corr_stms(const CorrArgs& a, CorrLds& L, PairLds
  * Bound by the STM of each round (half a period is about 30 attempts): with one
  * wave for it, run to its end in every round, 200 corrections took 3.32 ms (the
  * longest has 24 rounds of 100 us and nine STMs of 108 us after them; a usual
- * one five rounds of 148 us), now 2.52 ms.                                   */
+ * one five rounds of 148 us), now 2.41 ms.                                   */
 __global__ __launch_bounds__(256) void k_correct(CorrArgs a) {
     __shared__ CorrLds L;
     __shared__ PowTab powt;

@@ -27,8 +27,8 @@
  * (RowTab), but a wave holds four trajectories instead of eight.
  *
  * Measured against the form before (components in lanes 0..5, LDS swizzles,
- * IEEE divisions and branches): 1,024 x 2,000 RK8 steps 7.29 -> 3.81 ms (153
- * ns a stage, about 75 instructions of a wave alone on its SIMD), 500
+ * IEEE divisions and branches): 1,024 x 2,000 RK8 steps 7.29 -> 3.73 ms (150
+ * ns a stage, about 74 instructions of a wave alone on its SIMD), 500
  * manifold arcs 5.31 -> 3.36 ms (1.28 with group6_points), 32,768 event
  * searches 0.72 -> 0.59 ms.
  */
@@ -43,6 +43,11 @@ __device__ __forceinline__ double bperm(double v, int addr) {
     const int lo = __builtin_amdgcn_ds_bpermute(addr, __double2loint(v));
     const int hi = __builtin_amdgcn_ds_bpermute(addr, __double2hiint(v));
     return __hiloint2double(hi, lo);
+}
+
+/* v, negated where s has bit 31 set */
+__device__ __forceinline__ double xor_sign(double v, unsigned s) {
+    return __hiloint2double((int)((unsigned)__double2hiint(v) ^ s), __double2loint(v));
 }
 
 /* lane K (0..15) of each row, in every lane of the row */
@@ -176,7 +181,7 @@ struct Lanes6 {
                                  lane's quotient as the field writes it            */
     double c1;                /* the quotient's mass, 0 in lanes without one       */
     double c2;                /* factor of the velocity entry in the lane's row    */
-    unsigned long long sign;  /* bit 63: this lane's derivative is negated         */
+    unsigned sign;            /* bit 31: this lane's derivative is negated         */
     const PowTab* pt;         /* hh_pow's tables (an LDS copy)                     */
     int lane;
     DopRow tab;               /* filled for the 16-lane form's attempts (dop_setup) */
@@ -204,7 +209,7 @@ struct Lanes6 {
         b2 = l == 4 ? mu_ : -0.0;
         c1 = act ? (vel ? mu_ : one_mu) : 0.0;
         c2 = l < 3 ? 1.0 : (l == 4 ? 2.0 : (l == 5 ? -2.0 : (l == 6 ? -1.0 : 0.0)));
-        sign = (act && fwd == -1 && ((flip >> d) & 1ULL)) ? (1ULL << 63) : 0ULL;
+        sign = (act && fwd == -1 && ((flip >> d) & 1ULL)) ? 1u << 31 : 0u;
     }
 
     /* byte address of the lane of this group that holds component k */
@@ -270,7 +275,7 @@ struct Lanes6 {
         const double head = c2 * pv + (xy ? w : -0.0);
         double o = (head - q1) - q2;
         if constexpr (!FAST) o = act ? o : 0.0;   /* 0/0 and the like in idle lanes */
-        return __longlong_as_double(__double_as_longlong(o) ^ (long long)sign);
+        return xor_sign(o, sign);
     }
 
     __device__ __forceinline__ double rhs(double v) const {

@@ -23,11 +23,12 @@
  * general forms, from the flags both waves write beside the sums.
  *
  * Bound by the two instruction streams, which are about equally long: of the
- * 8,800 cycles of an attempt the state wave waits 950 for the other's last
- * stage and sums, the STM wave 550 for records.  One trajectory alone: 3.59 us
+ * 8,400 cycles of an attempt the state wave waits 950 for the other's last
+ * stage and sums, the STM wave 550 for records.  One trajectory alone: 3.42 us
  * an attempt (5.83 us with twelve quotients read back by readlane, IEEE
  * divisions, both roles in one stream and a barrier a stage; a barrier a stage
- * alone costs what the tags do, 3.56 us), 5.0 us in the one-wave form (6.75
+ * alone costs what the tags do; 3.59 us with selected powers, see quotient), 4.8
+ * us in the one-wave form (6.75
  * us).  262,144 uneven trajectories on the persistent kernel, whose heaviest
  * ones end in this form: 94 -> 59 ms.
  */
@@ -158,10 +159,10 @@ struct Pair42 : Var42 {
     template <bool FAST>
     __device__ __forceinline__ double rhs_form(double v, FastChk& c, int n) const {
         if constexpr (ROLE == 0) {
-            double w, u;
-            const double q = quotient<FAST>(v, c, w, u);
+            double w, u, pos;
+            const double q = quotient<FAST>(v, c, w, u, pos);
             hand_over(n, q, u);
-            double o = xor_sign(state_row<FAST>(v, q, w), sign);
+            double o = xor_sign(state_row<FAST>(v, q, w, pos), sign);
             /* the stores leave before the next stage begins */
             asm volatile("" : "+v"(o) : : "memory");
             return o;
@@ -176,12 +177,12 @@ struct Pair42 : Var42 {
             FastChk c;
             c.num(mu);
             c.num(mu2);
-            double w, u;
-            double q = quotient<true>(v, c, w, u);
+            double w, u, pos;
+            double q = quotient<true>(v, c, w, u, pos);
             const bool general = __any(left_range(c));
-            if (__builtin_expect(general, 0)) q = quotient<false>(v, c, w, u);
+            if (__builtin_expect(general, 0)) q = quotient<false>(v, c, w, u, pos);
             hand_over(n, q, u);
-            return xor_sign(state_row<false>(v, q, w), sign);
+            return xor_sign(state_row<false>(v, q, w, pos), sign);
         } else {
             return xor_sign(column<false>(v, n), sign);
         }
