@@ -497,15 +497,26 @@ __global__ __launch_bounds__(256) void k_rk_fixed6_group(
     if (p.act) yout[(size_t)d * n + i] = y;
 }
 
+/* This wave's SIMD as an index < SIMD_TAB, from the hardware id registers
+ * (XCC, shader engine, array, CU, SIMD).  Only used to find the other waves
+ * that share a SIMD; a wrong layout would cost time, never results.        */
+constexpr int SIMD_TAB = 65536;
+__device__ __forceinline__ int simd_key() {
+    const unsigned hw = __builtin_amdgcn_s_getreg((31 << 11) | 4);    /* HW_ID, 32 bits  */
+    const unsigned xcc = __builtin_amdgcn_s_getreg((3 << 11) | 20);   /* XCC_ID, 4 bits  */
+    const unsigned simd = (hw >> 4) & 3u, cu = (hw >> 8) & 15u, sh = (hw >> 12) & 1u,
+                   se = (hw >> 13) & 7u;
+    return (int)(((xcc & 15u) << 12) | (se << 9) | (sh << 8) | (cu << 4) | simd);
+}
+
+/* Trajectory i of k_dop853_run6 in this lane */
 template <bool GRID>
-__global__ __launch_bounds__(256) void k_dop853_run6(
-    int n, const double* __restrict__ mu, const double* __restrict__ t0a,
+__device__ __forceinline__ void run6_lane(
+    int i, int n, const double* __restrict__ mu, const double* __restrict__ t0a,
     const double* __restrict__ tfa, StepParams sp, int fwd, unsigned long long flip,
     const double* __restrict__ y0, double* __restrict__ yout, int m,
     const double* __restrict__ teval, int* __restrict__ status, int* __restrict__ nacc,
     int* __restrict__ nrej) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
     Lane6 p;
     p.mu = mu[i];
     p.flipbits = lane_flip_bits(fwd, flip, 0, false);
@@ -537,6 +548,72 @@ __global__ __launch_bounds__(256) void k_dop853_run6(
     if (status) status[i] = s.status;
     if (nacc) nacc[i] = s.nacc;
     if (nrej) nrej[i] = s.nrej;
+}
+
+template <bool GRID>
+__global__ __launch_bounds__(256) void k_dop853_run6(
+    int n, const double* __restrict__ mu, const double* __restrict__ t0a,
+    const double* __restrict__ tfa, StepParams sp, int fwd, unsigned long long flip,
+    const double* __restrict__ y0, double* __restrict__ yout, int m,
+    const double* __restrict__ teval, int* __restrict__ status, int* __restrict__ nacc,
+    int* __restrict__ nrej) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    run6_lane<GRID>(i, n, mu, t0a, tfa, sp, fwd, flip, y0, yout, m, teval, status, nacc, nrej);
+}
+
+/* End states of many trajectories.  A wave lasts as long as the longest of its
+ * 64 trajectories, so each workgroup deals its trajectories out in the order of
+ * their spans: every thread counts the spans below its own (BLOCK keys in LDS,
+ * about 4 us), and each wave takes the next 64.  A workgroup of 512 fills a CU
+ * (242 registers, two waves a SIMD); the two waves of a SIMD then take spans
+ * from opposite ends, by the SIMDs the waves find themselves on.  Which wave
+ * takes which trajectories decides only the time.
+ * 131,072 halo arcs with spans of 0.6 to 3: 1.92 -> 1.24 ms.               */
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_dop853_final6_spans(
+    int n, const double* __restrict__ mu, const double* __restrict__ t0a,
+    const double* __restrict__ tfa, StepParams sp, int fwd, unsigned long long flip,
+    const double* __restrict__ y0, double* __restrict__ yout, int* __restrict__ status,
+    int* __restrict__ nacc, int* __restrict__ nrej) {
+    constexpr int WAVES = BLOCK / 64;
+    __shared__ alignas(16) unsigned key[BLOCK];
+    __shared__ int order[BLOCK];
+    __shared__ int on_simd[4];
+    const int tid = threadIdx.x;
+    const int first = blockIdx.x * BLOCK;
+    const int i = first + tid;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (tid < 4) on_simd[tid] = 0;
+    /* the span's leading bits above the thread's number, so that keys differ;
+     * lanes past the end last                                               */
+    unsigned k = ~0u;
+    if (i < n) {
+        const double t0 = t0a[i], tf = tfa[i];
+        k = (tf > t0) ? __float_as_uint((float)(tf - t0)) : 0u;
+    }
+    k = (k & ~(unsigned)(BLOCK - 1)) | (unsigned)tid;
+    key[tid] = k;
+    __syncthreads();
+    const int simd = simd_key() & 3;
+    int nth = 0;
+    if ((tid & 63) == 0) nth = atomicAdd(&on_simd[simd], 1);
+    nth = __builtin_amdgcn_readfirstlane(nth);
+    int rank = 0;
+#pragma unroll 4
+    for (int j = 0; j < BLOCK; j += 4) {
+        const uint4 q = *(const uint4*)&key[j];
+        rank += (q.x < k) + (q.y < k) + (q.z < k) + (q.w < k);
+    }
+    order[rank] = tid;
+    __syncthreads();
+    int part = (blockIdx.x & 1) ? WAVES - 1 - wid : wid;
+    if (WAVES == 8 && on_simd[0] == 2 && on_simd[1] == 2 && on_simd[2] == 2 && on_simd[3] == 2)
+        part = nth == 0 ? simd : WAVES - 1 - simd;
+    const int mine = first + order[part * 64 + (tid & 63)];
+    if (mine >= n) return;
+    run6_lane<false>(mine, n, mu, t0a, tfa, sp, fwd, flip, y0, yout, 0, nullptr, status, nacc,
+                     nrej);
 }
 
 /* A caller's request to stop a loop early: with CANCEL set, the loops below
@@ -1487,18 +1564,6 @@ struct ResumeArgs {
                         reserves its SIMD (0 = never)                          */
 };
 
-/* This wave's SIMD as an index < SIMD_TAB, from the hardware id registers
- * (XCC, shader engine, array, CU, SIMD).  Only used to find the other waves
- * that share a SIMD; a wrong layout would cost time, never results.        */
-constexpr int SIMD_TAB = 65536;
-__device__ __forceinline__ int simd_key() {
-    const unsigned hw = __builtin_amdgcn_s_getreg((31 << 11) | 4);    /* HW_ID, 32 bits  */
-    const unsigned xcc = __builtin_amdgcn_s_getreg((3 << 11) | 20);   /* XCC_ID, 4 bits  */
-    const unsigned simd = (hw >> 4) & 3u, cu = (hw >> 8) & 15u, sh = (hw >> 12) & 1u,
-                   se = (hw >> 13) & 7u;
-    return (int)(((xcc & 15u) << 12) | (se << 9) | (sh << 8) | (cu << 4) | simd);
-}
-
 /* Reserves the wave's SIMD for a long run once the trajectory's projected
  * attempts, age * span / elapsed, reach r.exclusive (checked every 32
  * attempts): the other waves of the persistent kernel on that SIMD spill
@@ -2022,6 +2087,17 @@ StepParams make_sp(double rtol, double atol, double max_step, double min_step,
  * end states 0.64 and 0.62 ms at 8,192, 1.78 and 1.42 ms at 65,536.         */
 constexpr int ROW6_MAX = 4096;
 
+/* End states, one trajectory per lane, of more than SPANS6_MIN trajectories are
+ * dealt out by span: 131,072 spans of 0.6 to 3 take 1.24 ms and not 1.92,
+ * 262,144 2.2 and not 3.0.  It costs nothing there where all spans are equal
+ * (0.90 and 0.89 ms, 1.41 and 1.45 ms).  Fewer trajectories, less than three
+ * waves to two SIMDs, keep workgroups of 128: with 256 the CUs are loaded
+ * unevenly, and 81,920 equal spans take 0.86 ms and not 0.81 (0.88 with 512).
+ * From SPANS6_CU to SPANS6_CU_MAX workgroups of 512 have each its own CU:
+ * 114,688 spans of 0.6 to 3 take 1.28 ms with 512, 1.42 with 256, equal ones
+ * 0.89 either way (98,304 equal ones 0.88 and 0.85).                        */
+constexpr int SPANS6_MIN = 98304, SPANS6_CU = 114688, SPANS6_CU_MAX = 131072;
+
 template <class M>
 void launch_rk_fixed(int n, int dim, const double* mu, const double* t0p,
                             const double* tfp, int steps, const double* t_vals, int fwd,
@@ -2228,12 +2304,24 @@ int hh_dop853_final(int n, int dim, const double* mu, const double* t0, const do
     if (dim == 6) {
         if (variant != HH_VARIANT_PLAIN && variant != HH_VARIANT_WIDE)
             return fail(HH_ERR_ARGS, "hh_dop853_final: dim 6 supports the plain and wide variants");
+        const bool by_span = variant != HH_VARIANT_WIDE && block <= 0 && n > SPANS6_MIN;
         if (block <= 0) block = 128;
         if (block > 256 || block % 64) return fail(HH_ERR_ARGS, "hh_dop853_final: block must be 64..256, multiple of 64");
         if (variant == HH_VARIANT_WIDE)
             return launch_run6_group<false>(n, mu, t0, tf, sp, fwd, flip_mask, y0, y_out, 0,
                                             nullptr, status, n_acc, n_rej, block, st,
                                             "hh_dop853_final(6, wide) launch");
+        if (by_span) {
+            if (n >= SPANS6_CU && n <= SPANS6_CU_MAX)
+                hipLaunchKernelGGL(k_dop853_final6_spans<512>, dim3(blocks_for(n, 512)), dim3(512),
+                                   0, st, n, mu, t0, tf, sp, fwd, flip_mask, y0, y_out, status,
+                                   n_acc, n_rej);
+            else
+                hipLaunchKernelGGL(k_dop853_final6_spans<256>, dim3(blocks_for(n, 256)), dim3(256),
+                                   0, st, n, mu, t0, tf, sp, fwd, flip_mask, y0, y_out, status,
+                                   n_acc, n_rej);
+            return check_launch("hh_dop853_final(6) launch");
+        }
         hipLaunchKernelGGL(k_dop853_run6<false>, dim3(blocks_for(n, block)), dim3(block), 0, st, n,
                            mu, t0, tf, sp, fwd, flip_mask, y0, y_out, 0, (const double*)nullptr,
                            status, n_acc, n_rej);
