@@ -137,7 +137,7 @@ def rk_fixed(mu, y0, t0, tf, steps: int, *, order: int = 8, dim: int = 6, t_vals
     grid states as an (n, steps, dim) view, and with ``return_derivatives``
     (which implies the grid) also the derivative at every grid state, as
     _integrate_fixed_rk returns them.  For dim 6, ``variant`` "wide"
-    integrates one trajectory per 8-lane group (one component per lane, the
+    integrates one per group of 8 or 16 lanes (a component a lane, the
     latency form), "plain" one per lane; "auto" takes "wide" up to 65,536
     trajectories.  Both give the same bits.
     """
@@ -279,9 +279,9 @@ def _auto_variant(dim: int, n: int) -> str:
     """Layout of a final-value batch the caller leaves open.  6-d: lane groups
     up to 65,536 trajectories, one per lane beyond.  42-d: two waves per
     trajectory up to 4,096, where they fill the GPU (STMs of dispersed halo
-    states, pair / work-stealing / plain: 0.47 / 1.05 / 1.21 ms at 256, 1.42 /
-    1.55 / 1.79 ms at 4,096, 2.36 / 1.49 / 1.92 ms at 8,192), work stealing
-    beyond (2.7 against 5.8 ms at 65,536; 52 against 97 ms for uneven planar
+    states, pair / work-stealing / plain: 0.40 / 1.02 / 1.13 ms at 256, 1.29 /
+    1.57 / 1.64 ms at 4,096, 2.24 / 1.46 / 1.72 ms at 8,192), work stealing
+    beyond (2.6 against 5.5 ms at 65,536; 46 against 85 ms for uneven planar
     states, whose longest trajectories end in a wave of their own)."""
     if dim == 6:
         return "wide" if n <= 65536 else "plain"
@@ -358,8 +358,9 @@ def dop853_final(mu, y0, t0, tf, *, dim: int = 6, rtol: float = 1e-12, atol: flo
     """
     if variant == "auto":
         variant = _auto_variant(dim, 1 if np.ndim(y0) < 2 else len(y0))
-    b = prepare_final(mu, y0, t0, tf, dim,
-                      order="span" if variant.startswith("persistent") else None)
+    # the hand-out order is a matter of time only: no sort goes into a graph
+    by_span = variant.startswith("persistent") and not torch.cuda.is_current_stream_capturing()
+    b = prepare_final(mu, y0, t0, tf, dim, order="span" if by_span else None)
     launch_final(b, rtol=rtol, atol=atol, max_step=max_step, min_step=min_step,
                  max_steps=max_steps, forward=forward, flip_indices=flip_indices, variant=variant,
                  block=block, grid=grid, stream=stream)
@@ -382,7 +383,7 @@ def dop853_grid(mu, y0, t0, tf, m: int, *, dim: int = 6, t_eval=None, rtol: floa
     """States at the m points of numpy.linspace(t0, tf, m) -- or at the explicit
     times ``t_eval`` shared by all trajectories -- as the reference's
     dense-output phase produces them (rk.py:2497-2543).  ``variant`` "wide"
-    (dim 6 only) integrates one trajectory per 8-lane group; "auto" takes it
+    (dim 6 only) integrates one per group of 8 or 16 lanes; "auto" takes it
     for dim 6 up to 65,536 trajectories."""
     lib = _lib.load()
     y = _soa(y0, dim)
@@ -418,7 +419,7 @@ def dop853_event(mu, y0, t0, tmax, *, ev_index: int = 1, ev_offset: float = 0.0,
     """DOP853 until the first crossing of y[ev_index] = ev_offset (rk.py:2678-2803).
 
     ``variant`` "plain" integrates one trajectory per lane (throughput);
-    "wide" one per 8-lane group, one component per lane (about 2.5x shorter
+    "wide" one per group of 8 or 16 lanes, a component a lane (much shorter
     per trajectory; faster overall up to tens of thousands of trajectories);
     "auto" picks "wide" up to 65,536 trajectories.  All give the same bits."""
     lib = _lib.load()

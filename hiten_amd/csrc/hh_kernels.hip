@@ -3,8 +3,9 @@
  * Kernels (gfx950, wave64):
  *   k_rk_fixed6<M>      fixed-step RK of tableau M (RK4, RK6, RK8), 6-d, one
  *                       trajectory per lane (integrators/rk.py:531-588 over
- *                       numpy.linspace grid); k_rk_fixed6_group per 8-lane
- *                       group, k_rk_fixed42 on the 42-d variational system
+ *                       numpy.linspace grid); k_rk_fixed6_group per group
+ *                       of 8 or 16 lanes, k_rk_fixed42 on the 42-d
+ *                       variational system
  *   k_dop853_final6     DOP853 to t_f, 6-d, one trajectory per lane; the
  *                       returned state is the dense-output value at t_f
  *                       (rk.py:2375-2549 with t_eval = [t0, tf])
@@ -2483,9 +2484,9 @@ int hh_dop853_final_static(int n, int dim, const double* mu, const double* t0, c
 /* Up to this many 42-d trajectories a grid is formed one trajectory per
  * two-wave workgroup (Pair42, two waves a SIMD), more one per 8-lane group
  * (Lane42).  Pair against lanes, halo orbits over a period: one orbit x 1,000
- * points 0.43 and 1.33 ms, 200 x 200 points 0.47 and 1.11 ms, 1,024 x 2
- * points 0.48 and 0.65 ms, 1,024 x 1,000 0.70 and 1.79 ms; 2,048 x 2 points
- * 0.89 and 0.66 ms, 2,048 x 1,000 1.38 and 1.78 ms.                         */
+ * points 0.35 and 1.33 ms, 200 x 200 points 0.36 and 1.11 ms, 1,024 x 2
+ * points 0.40 and 0.65 ms, 1,024 x 1,000 0.61 and 1.79 ms; 2,048 x 2 points
+ * 0.75 and 0.60 ms, 2,048 x 1,000 1.21 and 1.65 ms.                         */
 constexpr int PAIR_GRID_MAX = 1024;
 
 int hh_dop853_grid(int n, int dim, const double* mu, const double* t0, const double* tf, int m,

@@ -98,7 +98,7 @@ int hh_get_tuning(hh_tuning_t* t);
  *   traj_out   : [steps][dim][n] every grid state, or NULL
  *   variant    : HH_VARIANT_PLAIN (one trajectory per lane, or per 8-lane
  *                group for dim 42) or HH_VARIANT_WIDE (dim 6: one
- *                trajectory per 8-lane group, one component per lane: the
+ *                trajectory per group of 8 or 16 lanes, a component a lane: the
  *                latency form for small batches); same results either way
  *   block      : threads per block (64..256, 0 = default)              */
 int hh_rk8_fixed(int n, int dim, const double* mu, const double* t0, const double* tf, int steps,
@@ -160,7 +160,7 @@ int hh_rk_fixed_event(int order, int n, const double* mu, const double* t0, cons
  *                move to the resume queue), or
  *                HH_VARIANT_WIDE (dim 42: one trajectory per wave, one
  *                component per lane, from the start; dim 6: one trajectory
- *                per 8-lane group, one component per lane: the latency
+ *                per group of 8 or 16 lanes, a component a lane: the latency
  *                forms for batches smaller than the GPU's wave slots) or
  *                HH_VARIANT_PAIR (dim 42: one trajectory per 128-thread
  *                workgroup, the state and the STM integrated by two waves
