@@ -1,6 +1,6 @@
 /* hh_correct.h -- the device-resident single-shooting corrector.
  *
- * One workgroup of four waves runs one correction's whole Newton-Armijo
+ * One workgroup of three waves runs one correction's whole Newton-Armijo
  * loop (the row functions of hh_newton.h: corrector/backends/newton.py:
  * 39-143, stepping/armijo.py:58-164) without returning to the host:
  *
@@ -14,9 +14,9 @@
  *              line search's outcome (a trial accepted with all trials
  *              before it known), the groups still on later trials stop;
  *   Jacobian   Phi(t_event) from [I | x] (corrector/operators.py:298-307,
- *              437-452) in the Pair42 layout on waves 2 and 3 -- for the
- *              round's state 0 speculatively, while the groups search for
- *              its crossing (corr_spec_stm) -- then the Halo term
+ *              437-452) in the Wave42 layout on wave 2 -- for the round's
+ *              state 0 speculatively, while the groups search for its
+ *              crossing (corr_spec_stm) -- then the Halo term
  *              (services/orbits.py:917-947);
  *   step       the 2x2 dense solve with its regularisation
  *              (corrector/backends/base.py:187-245), as NumPy's LAPACK
@@ -71,7 +71,7 @@ struct CorrLds {
     double spec_phi[42];  /* Phi of the round's state 0, integrated speculatively  */
     double spec_tf;       /* its event time, once known                         */
     int spec_known;       /* set when state 0's residual is in                  */
-    int spec_ok;          /* state 0's STM is wanted (corr_wants_stm)            */
+    int spec_ok;          /* state 0 crossed the section                        */
     int spec_valid;       /* spec_phi holds Phi(spec_tf) of state 0             */
     int use_spec;         /* this round's STM is state 0's: take spec_phi       */
     int n_eval;   /* states to evaluate this round: 1 (residual) or nal (trials) */
@@ -257,7 +257,7 @@ __device__ __forceinline__ void corr_try_decide(CorrLds& L, int n_eval) {
                                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-/* Phi(t_event) of the round's state 0 in the Pair42 layout, begun before
+/* Phi(t_event) of the round's state 0 in the Wave42 layout, begun before
  * t_event is known.  DOP853's steps do not depend on the end time until a
  * step would pass it (integrators/utils.py:205-207 clips that step; the
  * initial step, utils.py:149-157, ignores it), so the integration runs
@@ -267,10 +267,10 @@ __device__ __forceinline__ void corr_try_decide(CorrLds& L, int n_eval) {
  * It keeps the starting state and the last two accepted states with the
  * furthest time their attempts reached; if an older state's attempts
  * reached t_event it starts over.  Returns 1 with this lane's component of
- * the final state in `out`, 0 when no STM of state 0 is needed, -1 when it gives up (a non-finite error norm before t_event is
+ * the final state in `out`, 0 when state 0 has no crossing (no STM is
+ * needed), -1 when it gives up (a non-finite error norm before t_event is
  * known, or the attempt cap): the caller then integrates as usual.       */
-template <class WL>
-__device__ __forceinline__ int corr_spec_stm(const WL& W, const StepParams& sp, double y0,
+__device__ __forceinline__ int corr_spec_stm(const Wave42& W, const StepParams& sp, double y0,
                                              CorrLds& L, double& out, int& nacc_out) {
     double k[DOP_K];
 #pragma unroll
@@ -291,7 +291,9 @@ __device__ __forceinline__ int corr_spec_stm(const WL& W, const StepParams& sp, 
     double older = -INFINITY;
     const long long cap = sp.max_steps;
     for (;;) {
-        if (W.seen) break;   /* spec_known, as both waves saw it in the last norm */
+        if (__builtin_amdgcn_readfirstlane(__hip_atomic_load(
+                &L.spec_known, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP)))
+            break;
         if (na + nr >= cap) return -1;
         const double hh = clamp_step(h, sp.max_step, sp.min_step);
         rB = (t + hh > rB) ? t + hh : rB;
@@ -315,7 +317,7 @@ __device__ __forceinline__ int corr_spec_stm(const WL& W, const StepParams& sp, 
             nr += 1;
         }
     }
-    if (!__builtin_amdgcn_readfirstlane(L.spec_ok)) return 0;
+    if (!L.spec_ok) return 0;
     const double tf = L.spec_tf;
     if (isclose(0.0, tf) || !((0.0 - tf) * 1.0 < 0.0)) {
         /* zero or reversed span: y0 unchanged (dynamics/base.py:421-424) */
@@ -339,10 +341,9 @@ __device__ __forceinline__ int corr_spec_stm(const WL& W, const StepParams& sp, 
     return 1;
 }
 
-/* Phi(tf) from y0, the end time known from the start (k_dop853_final42_pair's
- * loop).                                         */
-template <class WL>
-__device__ __forceinline__ void corr_stm(const WL& W, const StepParams& sp, double y0,
+/* Phi(tf) from y0 in the Wave42 layout, the end time known from the start
+ * (k_dop853_final42_wide's loop).                                         */
+__device__ __forceinline__ void corr_stm(const Wave42& W, const StepParams& sp, double y0,
                                          double tf, double& out, int& nacc) {
     WideFinal o;
     int status, nr;
@@ -354,8 +355,7 @@ __device__ __forceinline__ void corr_stm(const WL& W, const StepParams& sp, doub
 
 /* This lane's component of [I | state]: the identity block of Phi, then
  * the full 6-d state of the controls q.                                   */
-template <class WL>
-__device__ __forceinline__ double corr_stm_start(const WL& W, const hh::NewtonRow& w,
+__device__ __forceinline__ double corr_stm_start(const Wave42& W, const hh::NewtonRow& w,
                                                  const double* q) {
     if (!W.holds()) return W.idle();
     const int c = W.comp();
@@ -366,177 +366,29 @@ __device__ __forceinline__ double corr_stm_start(const WL& W, const hh::NewtonRo
     return v;
 }
 
-/* Whether the step that follows state 0's residual needs Phi at its event time:
- * not when it ends the Newton loop, nor when the line search turns it down.
- * Only a hint: an STM that turns out to be needed after all (the best of trials
- * that were all turned down) is integrated later.                          */
-__device__ __forceinline__ bool corr_wants_stm(const hh::NewtonRow& w, bool trials,
-                                               const double* xe) {
-    double r[2];
-    for (int q = 0; q < 2; ++q) r[q] = xe[w.res[q]] - w.tgt[q];
-    const double rn = hh::newton_inf_norm(r, 2);
-    if (rn < w.tol || w.k + (trials ? 1 : 0) >= w.max_att) return false;
-    return !trials || rn <= (1.0 - w.c * w.alpha[0]) * w.rn;
-}
-
-/* Waves 0 and 1: residuals and line-search trials, and thread 0's decisions */
-__device__ __forceinline__ void corr_searches(const CorrArgs& a, CorrLds& L, const PowTab* pt,
-                                              int tid) {
-    const int lane = tid & 63;
-    const int grp = tid >> 3;
-    const double mu = L.row.mu;
-    Group6 ga, ge;
-    ga.setup(lane, mu, L.row.fwd, a.x.flip_align, pt);
-    ge.setup(lane, mu, 1, 0ULL, pt);
-    for (;;) {
-        const int n_eval = L.n_eval;
-        const bool trials = L.row.stage == hh::NS_ARMIJO;
-        for (int j0 = 0; j0 < n_eval; j0 += CORR_GROUPS) {
-            const int j = j0 + grp;
-            if (j < n_eval) {
-                const double* q = trials ? L.row.trial[j] : L.row.x;
-                double y = 0.0;
-                if (ge.act) {
-                    y = L.row.base[ge.d];
-                    for (int c = 0; c < 2; ++c)
-                        if (L.row.ctrl[c] == ge.d) y = q[c];
-                }
-                int ok, steps;
-                double t, xe;
-                const bool in = corr_residual<true>(ga, ge, a.x, L.ev_index, y, ok, t, xe, steps,
-                                                    &L.decided);
-                if (in && ge.act) L.xe[j][ge.d] = xe;
-                /* this group's results, then its flags, then the scan */
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-                if (ge.d == 0) {
-                    atomicAdd(&L.steps, steps);
-                    if (in) {
-                        L.t[j] = t;
-                        L.ok[j] = ok;
-                    }
-                    if (j == 0) {
-                        L.spec_tf = t;
-                        L.spec_ok = in && ok && corr_wants_stm(L.row, trials, L.xe[0]);
-                    }
-                }
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-                if (ge.d == 0 && j == 0)
-                    __hip_atomic_store(&L.spec_known, 1, __ATOMIC_RELEASE,
-                                       __HIP_MEMORY_SCOPE_WORKGROUP);
-                if (in && ge.d == 0 && trials) {
-                    __hip_atomic_store(&L.known[j], 1, __ATOMIC_SEQ_CST,
-                                       __HIP_MEMORY_SCOPE_WORKGROUP);
-                    corr_try_decide(L, n_eval);
-                }
-            }
-            __syncthreads();
-            if (tid == 0) {
-                const int done_n = (j0 + CORR_GROUPS < n_eval) ? j0 + CORR_GROUPS : n_eval;
-                L.more = (trials && !hh::newton_armijo_decided(L.row, 2, done_n, &L.xe[0][0],
-                                                               L.ok)) ? 1 : 0;
-            }
-            __syncthreads();
-            if (!L.more) break;
-        }
-        if (tid == 0) {
-            int taken = 0;
-            if (L.row.stage == hh::NS_RESID)
-                hh::newton_residual(L.row, 2, L.t[0], L.xe[0], L.ok[0]);
-            else
-                taken = hh::newton_armijo(L.row, 2, 2, L.t, &L.xe[0][0], L.ok);
-            /* the STM this step needs is state 0's when state 0 is the next
-             * iterate: its speculative integration ended at the same event
-             * time                                                           */
-            L.use_spec = (L.row.stage == hh::NS_JAC) && taken == 0 && L.spec_valid;
-        }
-        __syncthreads();
-        if (L.row.stage == hh::NS_DONE) break;
-        __syncthreads();   /* the STM pair's Phi */
-        if (tid == 0) {
-            double J[4], r[2], d[2];
-            hh::newton_jacobian(L.row, 2, 2, L.use_spec ? L.spec_phi : L.phi, J, r, DevPow());
-            corr_solve2(J, r, d);
-            hh::newton_set_step(L.row, 2, d);
-            L.n_eval = L.row.nal;
-            L.decided = 0;
-            for (int j = 0; j < L.row.nal; ++j) L.known[j] = 0;
-            L.spec_known = 0;
-            L.spec_valid = 0;
-        }
-        __syncthreads();
-    }
-}
-
-/* Waves 2 and 3: the STMs, in the given role of the pair, through the same
- * barriers as the searches                                                  */
-template <int ROLE>
-__device__ __forceinline__ void corr_stms(const CorrArgs& a, CorrLds& L, PairLds* plds,
-                                          const PowTab* pt, int lane) {
-    Pair42<ROLE, true> W;
-    W.setup(lane, L.row.mu, 1, a.flip_stm, plds, pt);
-    W.watch = &L.spec_known;
-    for (;;) {
-        const int n_eval = L.n_eval;
-        for (int j0 = 0; j0 < n_eval; j0 += CORR_GROUPS) {
-            if (j0 == 0) {
-                const bool trials = L.row.stage == hh::NS_ARMIJO;
-                const double y0 = corr_stm_start(W, L.row, trials ? L.row.trial[0] : L.row.x);
-                double out = 0.0;
-                int na = 0;
-                const int r = corr_spec_stm(W, a.sp_stm, y0, L, out, na);
-                if (r == 1 && W.holds()) L.spec_phi[W.comp()] = out;
-                if (W.leader()) {
-                    L.spec_valid = (r == 1);
-                    atomicAdd(&L.steps, na);
-                }
-            }
-            __syncthreads();
-            __syncthreads();
-            if (!L.more) break;
-        }
-        __syncthreads();
-        if (L.row.stage == hh::NS_DONE) break;
-        if (!L.use_spec) {
-            /* Phi(t_event) from [I | x] */
-            double out;
-            int na;
-            corr_stm(W, a.sp_stm, corr_stm_start(W, L.row, L.row.x), L.row.t_ev, out, na);
-            if (W.holds()) L.phi[W.comp()] = out;
-            if (W.leader()) atomicAdd(&L.steps, na);
-        }
-        __syncthreads();
-        __syncthreads();
-    }
-}
-
-/* One correction per workgroup of four waves, one on each SIMD of a CU: waves 0
- * and 1 are the sixteen Group6 groups that evaluate residuals and line-search
- * trials, waves 2 and 3 integrate the STMs in the Pair42 layout -- in each
- * round speculatively, for the round's state 0 (the residual's state, or the
- * alpha = 1 trial, which is the next iterate in most steps) while the groups
- * search for the crossings, until state 0's residual shows whether its STM is
- * needed.  Thread 0 keeps the row in LDS and takes the decisions between
- * barriers; every branch the waves take on LDS values is read after a barrier,
- * so all threads meet every barrier.  Each loop ends: every integration is
- * bounded by max_steps and the Newton loop by max_attempts, the STM pair's
- * speculation ends when state 0's search publishes its event time, which the
- * first group always does, and the pair's waves wait only for each other's
- * part of the same norm or right-hand side.
- *
- * Bound by the STM of each round (half a period is about 30 attempts): with one
- * wave for it, run to its end in every round, 200 corrections took 3.32 ms (the
- * longest has 24 rounds of 100 us and nine STMs of 108 us after them; a usual
- * one five rounds of 148 us), now 2.41 ms.                                   */
-__global__ __launch_bounds__(256) void k_correct(CorrArgs a) {
+/* One correction per 192-thread workgroup: waves 0 and 1 are the sixteen
+ * Group6 groups that evaluate residuals and line-search trials, wave 2
+ * integrates the STMs in the Wave42 layout -- in each round speculatively,
+ * for the round's state 0 (the residual's state, or the alpha = 1 trial,
+ * which is the next iterate in most steps) while the groups search for
+ * the crossings.  Thread 0 keeps the row in LDS and takes the decisions
+ * between barriers; every branch the waves take on LDS values is read after
+ * a barrier, so all threads meet every barrier.  Each loop ends: every
+ * integration is bounded by max_steps and the Newton loop by max_attempts,
+ * and the STM wave's speculation ends when state 0's search publishes its
+ * event time, which the first group always does.                         */
+__global__ __launch_bounds__(192) void k_correct(CorrArgs a) {
     __shared__ CorrLds L;
     __shared__ PowTab powt;
-    __shared__ PairLds plds;
+    __shared__ StageRec rec, zero;
     const int i = blockIdx.x;
     const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int grp = tid >> 3;
     const int wid = __builtin_amdgcn_readfirstlane((int)(tid >> 6));
     if (i >= a.n) return;
     pow_tab_fill(&powt);
-    pair_lds_clear(plds);
+    wave_lds_clear(zero);
     if (tid == 0) {
         const hh_correction_t& pb = a.prob[i];
         L.fail = 1;
@@ -557,10 +409,113 @@ __global__ __launch_bounds__(256) void k_correct(CorrArgs a) {
         L.spec_valid = 0;
     }
     __syncthreads();
-    if (!__builtin_amdgcn_readfirstlane(L.fail)) {
-        if (wid == 2) corr_stms<0>(a, L, &plds, &powt, tid & 63);
-        else if (wid == 3) corr_stms<1>(a, L, &plds, &powt, tid & 63);
-        else corr_searches(a, L, &powt, tid);
+    if (!L.fail) {
+        const double mu = L.row.mu;
+        Group6 ga, ge;
+        ga.setup(lane, mu, L.row.fwd, a.x.flip_align, &powt);
+        ge.setup(lane, mu, 1, 0ULL, &powt);
+        Wave42 W;
+        W.setup(lane, mu, 1, a.flip_stm, &powt, &rec, &zero);
+        for (;;) {
+            /* the residual, or the line-search trials of the step; the STM
+             * wave meanwhile integrates state 0's STM                      */
+            const int n_eval = L.n_eval;
+            const bool trials = L.row.stage == hh::NS_ARMIJO;
+            for (int j0 = 0; j0 < n_eval; j0 += CORR_GROUPS) {
+                const int j = j0 + grp;
+                if (wid < 2 && j < n_eval) {
+                    const double* q = trials ? L.row.trial[j] : L.row.x;
+                    double y = 0.0;
+                    if (ge.act) {
+                        y = L.row.base[ge.d];
+                        for (int c = 0; c < 2; ++c)
+                            if (L.row.ctrl[c] == ge.d) y = q[c];
+                    }
+                    int ok, steps;
+                    double t, xe;
+                    const bool in = corr_residual<true>(ga, ge, a.x, L.ev_index, y, ok, t,
+                                                        xe, steps, &L.decided);
+                    if (in && ge.act) L.xe[j][ge.d] = xe;
+                    if (ge.d == 0) {
+                        atomicAdd(&L.steps, steps);
+                        if (in) {
+                            L.t[j] = t;
+                            L.ok[j] = ok;
+                        }
+                        if (j == 0) {
+                            L.spec_tf = t;
+                            L.spec_ok = in && ok;
+                        }
+                    }
+                    /* this group's results, then its flags, then the scan */
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+                    if (ge.d == 0 && j == 0)
+                        __hip_atomic_store(&L.spec_known, 1, __ATOMIC_RELEASE,
+                                           __HIP_MEMORY_SCOPE_WORKGROUP);
+                    if (in && ge.d == 0 && trials) {
+                        __hip_atomic_store(&L.known[j], 1, __ATOMIC_SEQ_CST,
+                                           __HIP_MEMORY_SCOPE_WORKGROUP);
+                        corr_try_decide(L, n_eval);
+                    }
+                } else if (wid == 2 && j0 == 0) {
+                    const double y0 = corr_stm_start(W, L.row, trials ? L.row.trial[0] : L.row.x);
+                    double out = 0.0;
+                    int na = 0;
+                    const int r = corr_spec_stm(W, a.sp_stm, y0, L, out, na);
+                    if (r == 1 && W.holds()) L.spec_phi[W.comp()] = out;
+                    if (lane == 0) {
+                        L.spec_valid = (r == 1);
+                        L.steps += na;
+                    }
+                }
+                __syncthreads();
+                if (tid == 0) {
+                    const int done_n = (j0 + CORR_GROUPS < n_eval) ? j0 + CORR_GROUPS : n_eval;
+                    L.more = (trials && !hh::newton_armijo_decided(L.row, 2, done_n, &L.xe[0][0],
+                                                                   L.ok)) ? 1 : 0;
+                }
+                __syncthreads();
+                if (!L.more) break;
+            }
+            if (tid == 0) {
+                int taken = 0;
+                if (L.row.stage == hh::NS_RESID)
+                    hh::newton_residual(L.row, 2, L.t[0], L.xe[0], L.ok[0]);
+                else
+                    taken = hh::newton_armijo(L.row, 2, 2, L.t, &L.xe[0][0], L.ok);
+                /* the STM this step needs is state 0's when state 0 is the
+                 * next iterate: its speculative integration ended at the
+                 * same event time                                            */
+                L.use_spec = (L.row.stage == hh::NS_JAC) && taken == 0 && L.spec_valid;
+            }
+            __syncthreads();
+            if (L.row.stage == hh::NS_DONE) break;
+            /* Phi(t_event) from [I | x] */
+            if (wid == 2) {
+                if (L.use_spec) {
+                    if (W.holds()) L.phi[W.comp()] = L.spec_phi[W.comp()];
+                } else {
+                    double out;
+                    int na;
+                    corr_stm(W, a.sp_stm, corr_stm_start(W, L.row, L.row.x), L.row.t_ev, out, na);
+                    if (W.holds()) L.phi[W.comp()] = out;
+                    if (lane == 0) L.steps += na;
+                }
+            }
+            __syncthreads();
+            if (tid == 0) {
+                double J[4], r[2], d[2];
+                hh::newton_jacobian(L.row, 2, 2, L.phi, J, r, DevPow());
+                corr_solve2(J, r, d);
+                hh::newton_set_step(L.row, 2, d);
+                L.n_eval = L.row.nal;
+                L.decided = 0;
+                for (int j = 0; j < L.row.nal; ++j) L.known[j] = 0;
+                L.spec_known = 0;
+                L.spec_valid = 0;
+            }
+            __syncthreads();
+        }
     }
     if (tid == 0) {
         hh_correction_result_t& o = a.res[i];

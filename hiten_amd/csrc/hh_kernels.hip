@@ -1394,7 +1394,7 @@ __global__ __launch_bounds__(BLOCK) void k_dop853_final42_wide(Final42Args a) {
 
 /* One trajectory per pair of waves (128-thread workgroup) from the start:
  * the state wave and the STM wave of Pair42 side by side on two SIMDs.  Both
- * waves take the same branches and so meet in the same norms.               */
+ * waves take the same branches and so meet the same barriers.               */
 template <bool GRID, int ROLE>
 __device__ __forceinline__ void pair_from_start(const Final42Args& a, PairLds* lds,
                                                 const PowTab* pt, int traj, int lane) {
@@ -1696,7 +1696,6 @@ __device__ __forceinline__ void run_pair(const Final42Args& a, const ResumeArgs&
     __builtin_amdgcn_s_setprio(3);
     wide_finish(a, P, ho.traj, y, k, ho.t, ho.tf, ho.h, ho.err_prev, ho.nacc, ho.nrej, hook);
     __builtin_amdgcn_s_setprio(0);
-    P.finish();
     if (P.leader()) atomicSub(&r.ctr[3], 1);
 }
 
@@ -1713,14 +1712,14 @@ __device__ __forceinline__ void run_pair(const Final42Args& a, const ResumeArgs&
  * Waves leave once every trajectory has finished; each trajectory is bounded
  * by max_steps and every pairing or wave-wide run finishes one, so every
  * wave leaves.  The only waits are the barriers of a pair (both waves reach
- * them), what its waves wait for from each other (hh_pair.h) and the wait for a
- * claimed resume slot, whose producer writes it right after claiming it.    */
+ * them) and the wait for a claimed resume slot, whose producer writes it
+ * right after claiming it.                                                 */
 template <int BLOCK, int WPE>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 void k_dop853_final42_resume(Final42Args a, ResumeArgs r) {
     static_assert(BLOCK == 128, "the pair form takes two waves per workgroup");
     __shared__ PairLds plds;
-    __shared__ StageRec rec[2], zero;
+    __shared__ StageRec rec[2];
     __shared__ PairHandoff ho;
     __shared__ int pair_state;
     __shared__ PowTab powt;
@@ -1731,7 +1730,6 @@ void k_dop853_final42_resume(Final42Args a, ResumeArgs r) {
     if (threadIdx.x == 0) pair_state = -1;
     pow_tab_fill(&powt);
     pair_lds_clear(plds);
-    wave_lds_clear(zero);
     __syncthreads();
     const int key = simd_key();
     Lane42 p;
@@ -1818,7 +1816,7 @@ void k_dop853_final42_resume(Final42Args a, ResumeArgs r) {
             if (!moved) traj = -1;
             const int tr = __builtin_amdgcn_readlane(traj, src);
             const double t0 = a.t0[tr];
-            run_wide(a, &powt, &rec[wid], &zero, lane, src, traj, p, s,
+            run_wide(a, &powt, &rec[wid], &plds.zero[0], lane, src, traj, p, s,
                      SimdReserve{r.simd_tab, key, r.exclusive, lane, t0, a.tf[tr] - t0, false});
             if (lane == 0) atomicSub(&r.ctr[3], 1);
             forget42(p, s, o);
@@ -2629,7 +2627,7 @@ int hh_correct(int n, const hh_correction_t* problems, hh_correction_result_t* r
     if (rc != HH_OK) return rc;
     a.sp_stm = make_sp(1e-12, 1e-12, 1e4, 10.0 * DBL_EPSILON, 1000000);
     a.flip_stm = ((1ULL << 42) - 1) & ~((1ULL << 36) - 1);   /* the state block */
-    hipLaunchKernelGGL(k_correct, dim3(n), dim3(256), 0, (hipStream_t)stream, a);
+    hipLaunchKernelGGL(k_correct, dim3(n), dim3(192), 0, (hipStream_t)stream, a);
     return check_launch("hh_correct launch");
 }
 
