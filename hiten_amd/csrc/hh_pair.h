@@ -21,11 +21,11 @@
  * general forms, from the flags both waves write beside the sums.
  *
  * Bound by the longer of the two instruction streams and the LDS round trip
- * and barrier of every stage.  One trajectory alone: 3.56 us an attempt (5.83
+ * and barrier of every stage.  One trajectory alone: 3.4 us an attempt (5.83
  * us with twelve quotients read back by readlane, IEEE divisions and both
  * roles in one stream; 4.22 us before each role had a stream of its own, 3.94
  * us before the state row hid the record's stores, 3.74 us before the step
- * controller lost its branches), 4.88 us in the one-wave form (6.75 us).
+ * controller lost its branches), 4.8 us in the one-wave form (6.75 us).
  * 262,144 uneven trajectories on the persistent kernel, whose heaviest ones
  * end in this form: 94 -> 59 ms.
  */

@@ -148,8 +148,8 @@ struct Var42 {
             const double he = 0.5 * e;
             /* a factor P or 1 instead of a choice between powers: exact where it
              * is 1, and eight instructions of 88 fewer with the choice of the
-             * scale in cr and pos in state_row (3.59 -> 3.42 us an attempt of
-             * a pair, 0.902 -> 0.854 ms one trajectory on one wave)             */
+             * scale in cr and pos in state_row (0.640 -> 0.606 ms a trajectory
+             * on a pair, 0.902 -> 0.854 ms on one wave)                        */
             const double m = p5 ? P : 1.0;
             const double base = m * P, be = __builtin_fma(m, P, -base);
             const double t = m * s;
