@@ -581,7 +581,11 @@ __device__ __forceinline__ double wave_prev(double v) {
  * and dt |d1| <= |g(k+2) - g(k)| as long as the four times do not decrease.
  * With D(k) = |g(k+1) - g(k)| these are at most D(k-1) + D(k) and D(k) +
  * D(k+1), no division needed; 0.15 > 4/27 and 1e-8 |g| leave more room than the
- * rounding of the evaluated values takes.  NaN fails the test.            */
+ * rounding of the evaluated values takes.  NaN fails the test.  Values below
+ * SYN_TINY stay in: the sign test of two values is their product (syn_crosses),
+ * which for two of one sign may round to 0, and 0 counts as a crossing.  From
+ * SYN_TINY on, with all values of the segment above 1e-8 SYN_TINY, it does not. */
+constexpr double SYN_TINY = 1e-150;
 __device__ __forceinline__ unsigned long long syn_suspects(const SynArgs& a, int N, int j, int lane,
                                                            double g, double t) {
     const bool pair = j >= 0 && j + 1 < N;
@@ -589,7 +593,7 @@ __device__ __forceinline__ unsigned long long syn_suspects(const SynArgs& a, int
     const unsigned long long rising = __ballot(!pair || t <= wave_next(t));
     const double A = __builtin_fabs(g);
     const bool clear = (A - D > 0.15 * ((D + D) + (wave_prev(D) + wave_next(D))) + 1e-8 * A) &&
-                       A >= a.tol_on;
+                       A >= a.tol_on && A >= SYN_TINY;
     return __ballot(!clear) | ~(rising & (rising << 1) & (rising >> 1));
 }
 
