@@ -89,6 +89,31 @@ def _soa(y0, dim: int) -> torch.Tensor:
     return y.t().contiguous()
 
 
+def _capturing(stream) -> bool:
+    with torch.cuda.stream(stream):
+        return torch.cuda.is_current_stream_capturing()
+
+
+def _launch_stream(stream, *tensors) -> int:
+    """Raw handle of the stream a kernel is launched on, the current one for
+    None.  Inputs are laid out, filled and sorted on the current stream:
+    another stream waits for that first, and the allocator is told that it uses
+    ``tensors``, so that none is handed out again while the kernel runs.  Where
+    only one of the two streams is being captured there is nothing to wait for:
+    the work of a graph has no order with work outside it."""
+    cur = torch.cuda.current_stream()
+    if stream is None or int(stream.cuda_stream) == int(cur.cuda_stream):
+        return int(cur.cuda_stream)
+    if not isinstance(stream, torch.cuda.Stream):
+        stream = torch.cuda.ExternalStream(int(stream.cuda_stream))
+    if _capturing(stream) == torch.cuda.is_current_stream_capturing():
+        stream.wait_stream(cur)
+    for t in tensors:
+        if t is not None:
+            t.record_stream(stream)
+    return int(stream.cuda_stream)
+
+
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
@@ -165,7 +190,8 @@ def rk_fixed(mu, y0, t0, tf, steps: int, *, order: int = 8, dim: int = 6, t_vals
                          _ptr(tv), int(forward), flip_mask(dim, flip_indices), _ptr(y), _ptr(out),
                          _ptr(traj), _ptr(der), {"plain": _lib.HH_VARIANT_PLAIN,
                                                  "wide": _lib.HH_VARIANT_WIDE}[variant],
-                         int(block), _lib.stream_handle(stream))
+                         int(block),
+                         _launch_stream(stream, mu_t, t0_t, tf_t, tv, y, out, traj, der))
     _lib.check(rc, "hh_rk_fixed")
     if return_derivatives:
         return out.t(), traj.permute(2, 0, 1), der.permute(2, 0, 1)
@@ -210,7 +236,7 @@ def rk_fixed_event(mu, y0, t0, tf, steps: int, *, order: int = 8, t_vals=None,
                                _ptr(tv), int(forward), flip_mask(6, flip_indices), int(ev_index),
                                float(ev_offset), int(direction), float(xtol), float(gtol), _ptr(y),
                                _ptr(hit), _ptr(th), _ptr(yh), _ptr(yl), int(block),
-                               _lib.stream_handle(stream))
+                               _launch_stream(stream, mu_t, t0_t, tf_t, tv, y, hit, th, yh, yl))
     _lib.check(rc, "hh_rk_fixed_event")
     return FixedEventResult(hit.bool(), th, yh.t(), yl.t())
 
@@ -309,7 +335,8 @@ def launch_final(b: FinalBatch, *, rtol: float = 1e-12, atol: float = 1e-12,
                              int(forward), flip_mask(b.dim, flip_indices), _ptr(b.y0), _ptr(b.y),
                              _ptr(b.status), _ptr(b.n_accepted), _ptr(b.n_rejected), var,
                              int(block), int(grid), ws, ws_bytes, _ptr(b.order),
-                             _lib.stream_handle(stream))
+                             _launch_stream(stream, b.mu, b.t0, b.tf, b.y0, b.y, b.status,
+                                            b.n_accepted, b.n_rejected, b.order, b.workspace))
     _lib.check(rc, "hh_dop853_final")
 
 
@@ -356,10 +383,16 @@ def dop853_final(mu, y0, t0, tf, *, dim: int = 6, rtol: float = 1e-12, atol: flo
     """Adaptive DOP853 to tf; the state returned is the dense-output value at tf
     (the last row of _propagate_dynsys(..., steps=2)).
     """
+    # a graph recorded on the launch stream alone keeps neither a workspace nor
+    # a hand-out order of this call's alive
+    captured = torch.cuda.is_current_stream_capturing()
+    apart = stream is not None and not captured and _capturing(stream)
     if variant == "auto":
         variant = _auto_variant(dim, 1 if np.ndim(y0) < 2 else len(y0))
+        if apart and variant == "persistent":
+            variant = "plain"
     # the hand-out order is a matter of time only: no sort goes into a graph
-    by_span = variant.startswith("persistent") and not torch.cuda.is_current_stream_capturing()
+    by_span = variant.startswith("persistent") and not captured and not apart
     b = prepare_final(mu, y0, t0, tf, dim, order="span" if by_span else None)
     launch_final(b, rtol=rtol, atol=atol, max_step=max_step, min_step=min_step,
                  max_steps=max_steps, forward=forward, flip_indices=flip_indices, variant=variant,
@@ -405,7 +438,8 @@ def dop853_grid(mu, y0, t0, tf, m: int, *, dim: int = 6, t_eval=None, rtol: floa
                             float(atol), float(max_step), float(min_step), int(max_steps),
                             int(forward), flip_mask(dim, flip_indices), _ptr(y), _ptr(out),
                             _ptr(status), _ptr(nacc), _ptr(nrej), var, int(block),
-                            _lib.stream_handle(stream))
+                            _launch_stream(stream, mu_t, t0_t, tf_t, te, y, out, status, nacc,
+                                           nrej))
     _lib.check(rc, "hh_dop853_grid")
     return GridResult(out, status, nacc, nrej)
 
@@ -440,7 +474,9 @@ def dop853_event(mu, y0, t0, tmax, *, ev_index: int = 1, ev_offset: float = 0.0,
                              int(forward), flip_mask(6, flip_indices), _ptr(y), _ptr(hit),
                              _ptr(th), _ptr(yh), _ptr(yl), _ptr(status), _ptr(nacc), _ptr(nrej),
                              {"plain": _lib.HH_VARIANT_PLAIN, "wide": _lib.HH_VARIANT_WIDE}[variant],
-                             int(block), _lib.stream_handle(stream))
+                             int(block),
+                             _launch_stream(stream, mu_t, t0_t, tm_t, y, hit, th, yh, yl, status,
+                                            nacc, nrej))
     _lib.check(rc, "hh_dop853_event")
     return EventResult(hit.bool(), th, yh.t(), yl.t(), status, nacc, nrej)
 
@@ -452,8 +488,8 @@ def eval_rhs(mu, y, dim: int = 6, stream=None) -> torch.Tensor:
     n = ys.shape[1]
     mu_t = _vec(mu, n, "mu")
     out = torch.empty_like(ys)
-    _lib.check(lib.hh_eval_rhs(n, dim, _ptr(mu_t), _ptr(ys), _ptr(out), _lib.stream_handle(stream)),
-               "hh_eval_rhs")
+    _lib.check(lib.hh_eval_rhs(n, dim, _ptr(mu_t), _ptr(ys), _ptr(out),
+                               _launch_stream(stream, mu_t, ys, out)), "hh_eval_rhs")
     return out.t()
 
 
@@ -465,6 +501,6 @@ def eval_math(x, y, stream=None) -> torch.Tensor:
     yt = _vec(y, len(x), "y")
     n = xt.shape[0]
     out = torch.empty((6, n), dtype=torch.float64, device=xt.device)
-    _lib.check(lib.hh_eval_math(n, _ptr(xt), _ptr(yt), _ptr(out), _lib.stream_handle(stream)),
-               "hh_eval_math")
+    _lib.check(lib.hh_eval_math(n, _ptr(xt), _ptr(yt), _ptr(out),
+                                _launch_stream(stream, xt, yt, out)), "hh_eval_math")
     return out

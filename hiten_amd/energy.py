@@ -68,7 +68,8 @@ def traj_filters(states, mu, stream=None):
     mu_t = batch._vec(mu, n, "mu")
     out = torch.empty((3, n), dtype=torch.float64, device=S.device)
     rc = lib.hh_traj_filters(n, m, batch._ptr(mu_t), batch._ptr(S), batch._ptr(out[0]),
-                             batch._ptr(out[1]), batch._ptr(out[2]), _lib.stream_handle(stream))
+                             batch._ptr(out[1]), batch._ptr(out[2]),
+                             batch._launch_stream(stream, mu_t, S, out))
     _lib.check(rc, "hh_traj_filters")
     return out[0], out[1], out[2]
 
