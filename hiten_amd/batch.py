@@ -89,8 +89,15 @@ def _soa(y0, dim: int) -> torch.Tensor:
     return y.t().contiguous()
 
 
+def _torch_stream(stream):
+    """A torch stream from any object with a ``cuda_stream`` handle."""
+    if isinstance(stream, torch.cuda.Stream):
+        return stream
+    return torch.cuda.ExternalStream(int(stream.cuda_stream))
+
+
 def _capturing(stream) -> bool:
-    with torch.cuda.stream(stream):
+    with torch.cuda.stream(_torch_stream(stream)):
         return torch.cuda.is_current_stream_capturing()
 
 
@@ -104,14 +111,29 @@ def _launch_stream(stream, *tensors) -> int:
     cur = torch.cuda.current_stream()
     if stream is None or int(stream.cuda_stream) == int(cur.cuda_stream):
         return int(cur.cuda_stream)
-    if not isinstance(stream, torch.cuda.Stream):
-        stream = torch.cuda.ExternalStream(int(stream.cuda_stream))
+    stream = _torch_stream(stream)
     if _capturing(stream) == torch.cuda.is_current_stream_capturing():
         stream.wait_stream(cur)
     for t in tensors:
         if t is not None:
             t.record_stream(stream)
     return int(stream.cuda_stream)
+
+
+def _flags(hit: torch.Tensor, stream) -> torch.Tensor:
+    """hit != 0, formed on the stream the search runs on."""
+    if stream is None:
+        return hit.bool()
+    with torch.cuda.stream(_torch_stream(stream)):
+        f = hit.bool()
+    f.record_stream(torch.cuda.current_stream())
+    return f
+
+
+def _await_stream(stream) -> None:
+    """The current stream waits for ``stream``, whose results this call reads."""
+    if stream is not None:
+        torch.cuda.current_stream().wait_stream(_torch_stream(stream))
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -238,7 +260,7 @@ def rk_fixed_event(mu, y0, t0, tf, steps: int, *, order: int = 8, t_vals=None,
                                _ptr(hit), _ptr(th), _ptr(yh), _ptr(yl), int(block),
                                _launch_stream(stream, mu_t, t0_t, tf_t, tv, y, hit, th, yh, yl))
     _lib.check(rc, "hh_rk_fixed_event")
-    return FixedEventResult(hit.bool(), th, yh.t(), yl.t())
+    return FixedEventResult(_flags(hit, stream), th, yh.t(), yl.t())
 
 
 @dataclass
@@ -478,7 +500,7 @@ def dop853_event(mu, y0, t0, tmax, *, ev_index: int = 1, ev_offset: float = 0.0,
                              _launch_stream(stream, mu_t, t0_t, tm_t, y, hit, th, yh, yl, status,
                                             nacc, nrej))
     _lib.check(rc, "hh_dop853_event")
-    return EventResult(hit.bool(), th, yh.t(), yl.t(), status, nacc, nrej)
+    return EventResult(_flags(hit, stream), th, yh.t(), yl.t(), status, nacc, nrej)
 
 
 def eval_rhs(mu, y, dim: int = 6, stream=None) -> torch.Tensor:

@@ -541,7 +541,9 @@ def correct_device(problems: Sequence[CorrectionProblem], stream=None) -> list[C
     rec = pack_problems(problems)
     prob = torch.from_numpy(rec.view(np.uint8)).to(dev)
     res = torch.zeros(n * RESULT_DTYPE.itemsize, dtype=torch.uint8, device=dev)
-    launch_device(prob.data_ptr(), res.data_ptr(), n, stream)
+    launch_device(prob.data_ptr(), res.data_ptr(), n,
+                  stream_handle=batch._launch_stream(stream, prob, res))
+    batch._await_stream(stream)
     host = res.cpu().numpy().view(RESULT_DTYPE)
     return results_from_records(host, problems)
 

@@ -240,8 +240,10 @@ def plane_crossing_device(mu, states, surface: _PlaneEvent, forward: int, window
                                      surface.index, surface.offset, ev_dir, 1e-12, 1e-12,
                                      float(window[0]), float(window[1]), float(fallback[0]),
                                      float(fallback[1]), ok.data_ptr(), t.data_ptr(),
-                                     y.data_ptr(), None, _lib.stream_handle(stream)),
+                                     y.data_ptr(), None,
+                                     batch._launch_stream(stream, mu_d, y0, ok, t, y)),
                "hh_plane_crossing")
+    batch._await_stream(stream)
     return ok.cpu().numpy().astype(bool), t.cpu().numpy(), y.cpu().numpy().T.copy()
 
 

@@ -145,11 +145,13 @@ def detect_arrays(times, states, *, normal, offset: float = 0.0, plane_coords=("
                 float(dedup_point_tol), int(max_hits_per_traj or 0), int(newton_max_iter),
                 int(out.t.shape[1]), batch._ptr(out.count), batch._ptr(out.t),
                 batch._ptr(out.x), batch._ptr(out.p))
+        used = (tm, ln, st, out.count, out.t, out.x, out.p) + ((ws,) if two_pass else ())
+        sh = batch._launch_stream(stream, *used)
         if two_pass:
-            rc = lib.hh_synodic_detect_ws(*args, ws.data_ptr(), wsb, _lib.stream_handle(stream))
+            rc = lib.hh_synodic_detect_ws(*args, ws.data_ptr(), wsb, sh)
             _lib.check(rc, "hh_synodic_detect_ws")
         else:
-            rc = lib.hh_synodic_detect(*args, _lib.stream_handle(stream))
+            rc = lib.hh_synodic_detect(*args, sh)
             _lib.check(rc, "hh_synodic_detect")
 
     while True:
@@ -159,6 +161,7 @@ def detect_arrays(times, states, *, normal, offset: float = 0.0, plane_coords=("
                         torch.empty((n, cap, 6), dtype=torch.float64, device=dev),
                         torch.empty((n, cap, 2), dtype=torch.float64, device=dev))
         launch(out)
+        batch._await_stream(stream)
         most = int(out.count.max().item()) if n else 0
         if most <= cap:
             out.relaunch = lambda: launch(out)

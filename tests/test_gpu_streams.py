@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 import torch
 
-from hiten_amd import batch, energy, workloads as W
+from hiten_amd import batch, corrector, energy, singlehit, synodic, workloads as W
 
 pytestmark = pytest.mark.gpu
 MU = W.MU_EM
@@ -36,6 +36,8 @@ CALLS = {
         MU, y, None, None, 0, t_eval=np.linspace(0.0, 0.3, 50), stream=s)),
     "grid42": (50, lambda y, tf, s: batch.dop853_grid(
         MU, _stm(y), 0.0, tf, 20, dim=42, stream=s)),
+    "event": (1000, lambda y, tf, s: batch.dop853_event(MU, y, 0.0, tf, stream=s)),
+    "rk8 event": (200, lambda y, tf, s: batch.rk_fixed_event(MU, y, 0.0, tf, 100, stream=s)),
     "rk8": (200, lambda y, tf, s: batch.rk_fixed(MU, y, 0.0, tf, 100, return_derivatives=True,
                                                  stream=s)),
     "field": (1000, lambda y, tf, s: batch.eval_rhs(MU, y, stream=s)),
@@ -63,6 +65,38 @@ def test_other_stream_waits_for_its_inputs(gpu, name):
         for g, w in zip(got, want):
             assert torch.equal(g.cpu(), w)
         del junk
+
+
+def _corrections(y, s):
+    ps = [corrector.halo_problem(MU, [0.8234, 0, 0.0224 + 1e-5 * i, 0, 0.1343, 0],
+                                 max_attempts=10) for i in range(5)]
+    return np.array([[*r.x_corrected, r.half_period, r.n_stm]
+                     for r in corrector.correct_device(ps, stream=s)])
+
+
+def _sections(y, s):
+    a = torch.linspace(0.0, 40.0, 900, dtype=y.dtype, device=y.device)
+    X = torch.sin(a)[None, :, None] + y[:, None, :]
+    r = synodic.detect_arrays(a, X, normal=synodic.axis_normal("y"), cap=2, stream=s)
+    torch.cuda.synchronize()                # the hits beyond the counts are not written
+    return np.array([[h.time for h in row] for row in synodic.hits_from_arrays(r)])
+
+
+def _crossings(y, s):
+    plane = singlehit._PlaneEvent("y", 0.0, None)
+    ok, t, x = singlehit.plane_crossing_device(MU, y.cpu().numpy(), plane, 1, (0.0, 3.1),
+                                               (1.4, 3.1), stream=s)
+    return np.column_stack([ok, t, x])
+
+
+@pytest.mark.parametrize("call", [_corrections, _sections, _crossings])
+def test_results_read_on_the_host_are_the_other_streams(gpu, call):
+    y = torch.as_tensor(W.planar_seeds(np.random.default_rng(2), 40), device=gpu)
+    want = call(y, None)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(DELAY)            # the kernel starts late
+    np.testing.assert_array_equal(call(y, side), want)
 
 
 def test_capture_on_another_stream_than_the_current(gpu):
