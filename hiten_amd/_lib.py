@@ -64,6 +64,8 @@ _SIGNATURES = {
                            _P, _P, _I, _P], _I),
     "hh_dop853_final": ([_I, _I, _P, _P, _P, _D, _D, _D, _D, _LL, _I, _ULL, _P, _P, _P, _P, _P,
                          _I, _I, _I, _P, _LL, _P, _P], _I),
+    "hh_dop853_final_bounded": ([_I, _I, _I, _P, _P, _P, _D, _D, _D, _D, _LL, _I, _ULL, _P, _P, _P,
+                                 _P, _P, _I, _I, _I, _P, _LL, _P, _P], _I),
     "hh_dop853_final_workspace": ([_I, _I, _I], _LL),
     "hh_dop853_final_static": ([_I, _I, _P, _P, _P, _D, _D, _D, _D, _LL, _I, _ULL, _P, _P, _P, _P,
                                 _P, _I, _I, _I, _P, _P], _I),

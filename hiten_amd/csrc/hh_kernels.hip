@@ -1537,8 +1537,9 @@ void k_dop853_final42_persist(Final42Args a) {
  * library on the stream before each launch):
  *   ctr[0] fresh-work counter        ctr[1] resume slots claimed (tail)
  *   ctr[2] resume slots taken (head) ctr[3] trajectories not yet finished
- *   ctr[4] spills that found no slot (an error that the capacity rules
- *          out; such a trajectory would end with status HH_STATUS_DROPPED)
+ *   ctr[4] trajectories given up: spills that found no slot (ruled out by
+ *          the capacity) and slots whose owner did not write them in time.
+ *          They end with status HH_STATUS_DROPPED
  *   ctr[5] slots taken by waves that hand their work away to sleep beside
  *          a reserved SIMD (at most SLEEP_BUDGET(n); past it they keep
  *          working instead)
@@ -1555,6 +1556,19 @@ void k_dop853_final42_persist(Final42Args a) {
 constexpr int RQ_CTR = 64;          /* ints reserved for the counters      */
 constexpr int SPILL_W = 89;
 
+/* Every wait of the scheduler is bounded by this many polls (r.wait_polls): a
+ * poll takes 1 to 3 us, so some seconds, while the longest wait a run without
+ * a fault makes is that of idle waves for the last trajectory (3.4 us an
+ * attempt).  A wave that gives a wait up loses nothing where others work on:
+ * an idle one leaves, a sleeper goes on beside the reserved SIMD's run.  Only
+ * a claimed resume slot that stays unwritten costs its trajectory.         */
+constexpr int WAIT_POLLS = 1 << 22;
+
+/* pair_state of a workgroup: no pair, the wave that claimed it, or this once
+ * one of its waves has left (set by compare-and-swap from NONE, so that a wave
+ * never leaves a partner that has claimed the pair)                         */
+constexpr int PAIR_NONE = -1, PAIR_ALONE = -2;
+
 struct ResumeArgs {
     int* ctr;
     int* rq;
@@ -1563,7 +1577,22 @@ struct ResumeArgs {
     int* simd_tab;   /* SIMD_TAB ints: nonzero = that SIMD is reserved         */
     int exclusive;   /* projected attempts from which a wave-wide or pair run
                         reserves its SIMD (0 = never)                          */
+    int wait_polls;  /* bound of every wait, WAIT_POLLS                        */
 };
+
+/* Reset of a launch.  Every trajectory counts as dropped until its results are
+ * stored, so one that the scheduler gave up says so.                        */
+__global__ void k_resume_reset(ResumeArgs r, int n, int* status, int* nacc, int* nrej) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < RQ_CTR) r.ctr[i] = (i == 3) ? n : 0;
+    if (i < r.cap) r.rq[i] = -1;
+    if (i < SIMD_TAB) r.simd_tab[i] = 0;
+    if (i < n) {
+        if (status) status[i] = ST_DROPPED;
+        if (nacc) nacc[i] = 0;
+        if (nrej) nrej[i] = 0;
+    }
+}
 
 /* Reserves the wave's SIMD for a long run once the trajectory's projected
  * attempts, age * span / elapsed, reach r.exclusive (checked every 32
@@ -1710,10 +1739,11 @@ __device__ __forceinline__ void run_pair(const Final42Args& a, const ResumeArgs&
  * compare-and-swap), both waves spill what they hold and meet at a barrier;
  * a wave that finds its partner's claim joins it at its next iteration.
  * Waves leave once every trajectory has finished; each trajectory is bounded
- * by max_steps and every pairing or wave-wide run finishes one, so every
- * wave leaves.  The only waits are the barriers of a pair (both waves reach
- * them) and the wait for a claimed resume slot, whose producer writes it
- * right after claiming it.                                                 */
+ * by max_steps and every pairing or wave-wide run finishes one.  Waits: the
+ * barriers of a pair, which both waves reach, as none leaves while the other
+ * has claimed it; and, each bounded by r.wait_polls, the wait of idle waves for
+ * the end, the sleep beside a reserved SIMD and the wait for a claimed resume
+ * slot, whose producer writes it right after claiming it.                  */
 template <int BLOCK, int WPE>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 void k_dop853_final42_resume(Final42Args a, ResumeArgs r) {
@@ -1727,7 +1757,7 @@ void k_dop853_final42_resume(Final42Args a, ResumeArgs r) {
     const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int b = lane & 7;
     const int grp = lane >> 3;
-    if (threadIdx.x == 0) pair_state = -1;
+    if (threadIdx.x == 0) pair_state = PAIR_NONE;
     pow_tab_fill(&powt);
     pair_lds_clear(plds);
     __syncthreads();
@@ -1739,6 +1769,8 @@ void k_dop853_final42_resume(Final42Args a, ResumeArgs r) {
     int traj = -1;
     bool fresh_done = false;  /* the fresh counter has passed n                */
     bool queue_dry = false;   /* the last look at the resume queue found it empty */
+    bool awake = false;       /* gave a sleep up: reservations no longer bind     */
+    int idle = 0;             /* looks in a row that found nothing to do           */
     s.done = true;
     for (;;) {
         /* heavy trajectories (projected attempts = age * span / elapsed time):
@@ -1764,9 +1796,10 @@ void k_dop853_final42_resume(Final42Args a, ResumeArgs r) {
         int join = 0;
         if (hm) {
             int old = 0;
-            if (lane == 0) old = atomicCAS(&pair_state, -1, wid);
+            if (lane == 0) old = atomicCAS(&pair_state, PAIR_NONE, wid);
             old = __builtin_amdgcn_readfirstlane(__shfl(old, 0));
-            if (old == -1) owner_src = __ffsll((long long)hm) - 1;
+            if (old == PAIR_NONE) owner_src = __ffsll((long long)hm) - 1;
+            else if (old == PAIR_ALONE) heavy = heavy || huge;
             else join = 1;
         } else {
             join = __builtin_amdgcn_readfirstlane(
@@ -1802,7 +1835,7 @@ void k_dop853_final42_resume(Final42Args a, ResumeArgs r) {
             else run_pair<1>(a, r, ho, &plds, &powt, lane, key);
             forget42(p, s, o);
             __syncthreads();
-            if (threadIdx.x == 0) pair_state = -1;
+            if (threadIdx.x == 0) pair_state = PAIR_NONE;
             __syncthreads();
             continue;
         }
@@ -1825,7 +1858,7 @@ void k_dop853_final42_resume(Final42Args a, ResumeArgs r) {
         }
         /* a long run holds this SIMD: hand this wave's work to the others and
          * sleep until it is released (or a pair claim or the end wakes it) */
-        bool sleep = r.exclusive > 0 &&
+        bool sleep = r.exclusive > 0 && !awake &&
             __builtin_amdgcn_readfirstlane(__hip_atomic_load(&r.simd_tab[key], __ATOMIC_RELAXED,
                                                              __HIP_MEMORY_SCOPE_AGENT)) != 0;
         if (sleep && live) {
@@ -1845,13 +1878,20 @@ void k_dop853_final42_resume(Final42Args a, ResumeArgs r) {
         if (sleep) {
             spill42(a, r, traj >= 0, traj, b, grp, lane, s);
             traj = -1;
+            int polls = 0;
             while (__builtin_amdgcn_readfirstlane(
                        __hip_atomic_load(&r.simd_tab[key], __ATOMIC_RELAXED,
                                          __HIP_MEMORY_SCOPE_AGENT)) != 0 &&
                    __hip_atomic_load(&r.ctr[3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) > 0 &&
                    __builtin_amdgcn_readfirstlane(__hip_atomic_load(
-                       &pair_state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) < 0)
+                       &pair_state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) < 0) {
+                if (polls >= r.wait_polls) {
+                    awake = true;
+                    break;
+                }
+                ++polls;
                 __builtin_amdgcn_s_sleep(64);
+            }
             continue;
         }
         /* refill: the resume queue first, then fresh work; a wave that still
@@ -1882,13 +1922,22 @@ void k_dop853_final42_resume(Final42Args a, ResumeArgs r) {
                 int id = -1;
                 if (b == 0) {
                     /* the producer claimed this slot and writes it next */
-                    while ((id = __hip_atomic_load(&r.rq[rbase + rank], __ATOMIC_ACQUIRE,
-                                                   __HIP_MEMORY_SCOPE_AGENT)) < 0)
+                    for (int polls = 0;; ++polls) {
+                        id = __hip_atomic_load(&r.rq[rbase + rank], __ATOMIC_ACQUIRE,
+                                               __HIP_MEMORY_SCOPE_AGENT);
+                        if (id >= 0 || polls >= r.wait_polls) break;
                         __builtin_amdgcn_s_sleep(2);
+                    }
+                    if (id < 0) {   /* given up: its trajectory stays dropped */
+                        atomicAdd(&r.ctr[4], 1);
+                        atomicSub(&r.ctr[3], 1);
+                    }
                 }
                 traj = __shfl(id, grp * 8);
-                resume42(a, r, traj, b, p, s);
-                o.init(s.y);
+                if (traj >= 0) {
+                    resume42(a, r, traj, b, p, s);
+                    o.init(s.y);
+                }
             }
             const bool want = (traj < 0) && !fresh_done;
             const unsigned long long m = __ballot(want && b == 0);
@@ -1928,9 +1977,18 @@ void k_dop853_final42_resume(Final42Args a, ResumeArgs r) {
         }
         const unsigned long long fm = __ballot(finished && b == 0);
         if (fm && lane == 0) atomicSub(&r.ctr[3], __popcll(fm));
-        if (!__any(traj >= 0)) {
-            if (__hip_atomic_load(&r.ctr[3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <= 0)
-                break;
+        if (__any(traj >= 0)) {
+            idle = 0;
+        } else {
+            if (idle >= r.wait_polls ||
+                __builtin_amdgcn_readfirstlane(__hip_atomic_load(
+                    &r.ctr[3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) <= 0) {
+                /* unless the partner has claimed the pair: then it is joined */
+                int old = PAIR_NONE;
+                if (lane == 0) old = atomicCAS(&pair_state, PAIR_NONE, PAIR_ALONE);
+                if (__builtin_amdgcn_readfirstlane(__shfl(old, 0)) < 0) break;
+            }
+            ++idle;
             __builtin_amdgcn_s_sleep(8);
         }
     }
@@ -2292,7 +2350,21 @@ int hh_dop853_final(int n, int dim, const double* mu, const double* t0, const do
                     double* y_out, int* status, int* n_acc, int* n_rej, int variant, int block,
                     int grid, void* workspace, long long workspace_bytes, const int* order,
                     void* stream) {
+    return hh_dop853_final_bounded(WAIT_POLLS, n, dim, mu, t0, tf, rtol, atol, max_step, min_step,
+                                   max_steps, fwd, flip_mask, y0, y_out, status, n_acc, n_rej,
+                                   variant, block, grid, workspace, workspace_bytes, order,
+                                   stream);
+}
+
+int hh_dop853_final_bounded(int wait_polls, int n, int dim, const double* mu, const double* t0,
+                            const double* tf, double rtol, double atol, double max_step,
+                            double min_step, long long max_steps, int fwd,
+                            unsigned long long flip_mask, const double* y0, double* y_out,
+                            int* status, int* n_acc, int* n_rej, int variant, int block, int grid,
+                            void* workspace, long long workspace_bytes, const int* order,
+                            void* stream) {
     if (n < 0) return fail(HH_ERR_ARGS, "hh_dop853_final: n < 0");
+    if (wait_polls < 0) return fail(HH_ERR_ARGS, "hh_dop853_final_bounded: wait_polls < 0");
     if (n == 0) return HH_OK;
     if (dim != 6 && dim != 42) return fail(HH_ERR_ARGS, "hh_dop853_final: dim must be 6 or 42");
     if (!mu || !t0 || !tf || !y0 || !y_out) return fail(HH_ERR_ARGS, "hh_dop853_final: null pointer");
@@ -2378,6 +2450,7 @@ int hh_dop853_final(int n, int dim, const double* mu, const double* t0, const do
         r.spill = (double*)((char*)workspace + ws_align((long long)(RQ_CTR + r.cap) * 4));
         r.simd_tab = (int*)((char*)r.spill + ws_align((long long)SPILL_W * n * 8));
         r.exclusive = g_tuning.exclusive_projected;
+        r.wait_polls = wait_polls;
         const int wpe = g_tuning.waves_per_simd;
         int g = grid;
         if (g <= 0) {
@@ -2392,10 +2465,9 @@ int hh_dop853_final(int n, int dim, const double* mu, const double* t0, const do
          * workgroup's pair of waves, and with fewer workgroups than heavy
          * trajectories those would take the pairs one after the other      */
         if (g > n) g = n;
-        hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, st, r.ctr, 0, RQ_CTR);
-        hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, st, r.ctr + 3, n, 1);
-        hipLaunchKernelGGL(k_fill_int, dim3((r.cap + 255) / 256), dim3(256), 0, st, r.rq, -1, r.cap);
-        hipLaunchKernelGGL(k_fill_int, dim3(SIMD_TAB / 256), dim3(256), 0, st, r.simd_tab, 0, SIMD_TAB);
+        const int reset = r.cap > SIMD_TAB ? r.cap : SIMD_TAB;   /* cap > n */
+        hipLaunchKernelGGL(k_resume_reset, dim3((reset + 255) / 256), dim3(256), 0, st, r, n,
+                           status, n_acc, n_rej);
         if (wpe == 1)
             hipLaunchKernelGGL((k_dop853_final42_resume<128, 1>), dim3(g), dim3(128), 0, st, a, r);
         else

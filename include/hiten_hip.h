@@ -35,8 +35,9 @@ extern "C" {
 #define HH_STATUS_MAXSTEPS 1
 #define HH_STATUS_NONFINITE 2
 /* hh_dop853_final, variant HH_VARIANT_PERSISTENT_PAIR: a trajectory its
- * scheduler could not requeue (the workspace capacity rules this out; the
- * status exists so that such a loss is never silent).  y_out is undefined. */
+ * scheduler gave up: it found no room in the resume queue (the workspace
+ * capacity rules this out) or a wait for it ran out (hh_dop853_final_bounded).
+ * The status exists so that such a loss is never silent.  y_out is undefined. */
 #define HH_STATUS_DROPPED 4
 
 #define HH_VARIANT_PLAIN 0
@@ -182,6 +183,20 @@ int hh_dop853_final(int n, int dim, const double* mu, const double* t0, const do
                     const double* y0, double* y_out, int* status, int* n_acc, int* n_rej,
                     int variant, int block, int grid, void* workspace,
                     long long workspace_bytes, const int* order, void* stream);
+
+/* hh_dop853_final with the bound of the waits in HH_VARIANT_PERSISTENT_PAIR's
+ * scheduler stated: a wave that has polled wait_polls times (1 to 3 us each)
+ * for a resume slot gives that trajectory up (HH_STATUS_DROPPED), one that
+ * found no work as often leaves, one that slept as often beside a reserved
+ * SIMD goes on.  hh_dop853_final takes 2^22, some seconds.  The other variants
+ * wait for nothing.  No counterpart in the reference.                      */
+int hh_dop853_final_bounded(int wait_polls, int n, int dim, const double* mu, const double* t0,
+                            const double* tf, double rtol, double atol, double max_step,
+                            double min_step, long long max_steps, int fwd,
+                            unsigned long long flip_mask, const double* y0, double* y_out,
+                            int* status, int* n_acc, int* n_rej, int variant, int block, int grid,
+                            void* workspace, long long workspace_bytes, const int* order,
+                            void* stream);
 
 /* Bytes of workspace hh_dop853_final needs for (n, dim, variant): 0 for the
  * variants that need none.  No counterpart in the reference.              */
