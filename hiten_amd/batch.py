@@ -445,10 +445,11 @@ def dop853_grid(mu, y0, t0, tf, m: int, *, dim: int = 6, t_eval=None, rtol: floa
     n = y.shape[1]
     te = None
     if t_eval is not None:
-        te = _vec(t_eval, len(t_eval), "t_eval")
+        ts = t_eval if isinstance(t_eval, torch.Tensor) else np.asarray(t_eval, dtype=np.float64)
+        te = _vec(ts, len(t_eval), "t_eval")
         m = te.shape[0]
-        # the ends of host times are read on the host
-        t0, tf = float(t_eval[0]), float(t_eval[-1])
+        # the ends by position, those of host times without a wait for the device
+        t0, tf = float(ts[0]), float(ts[-1])
     mu_t, t0_t, tf_t = _vec(mu, n, "mu"), _vec(t0, n, "t0"), _vec(tf, n, "tf")
     out = torch.empty((n, int(m), dim), dtype=torch.float64, device=y.device)
     i32 = dict(dtype=torch.int32, device=y.device)
