@@ -446,36 +446,38 @@ def device_supported(p: CorrectionProblem, steps: Optional[dict] = None) -> bool
             and all(0 <= int(i) <= 5 for i in (*p.residual_indices, *p.control_indices))
             and int(p.event_index) in EVENT_PLANE):
         return False
-    if steps is None:
-        return line_search_steps(p) <= _JMAX
     key = (p.alpha_reduction, p.min_alpha)
+    if steps is None or not all(type(v) is float for v in key):
+        return line_search_steps(p) <= _JMAX
     if key not in steps:
         steps[key] = line_search_steps(p)
     return steps[key] <= _JMAX
 
 
 def _rows(values, shape) -> np.ndarray:
-    """Rows of ``shape`` from one value per problem (each broadcast to it)."""
+    """Rows of ``shape`` from one value per problem (each assigned to its row)."""
     try:
         a = np.array(values, dtype=float)
         if a.shape == (len(values), *shape):
             return a
     except ValueError:          # ragged: row by row
         pass
-    return np.array([np.broadcast_to(np.asarray(v, float), shape) for v in values])
+    a = np.empty((len(values), *shape))
+    for row, v in zip(a, values):
+        row[...] = np.asarray(v, float)
+    return a
 
 
 def pack_problems(problems: Sequence[CorrectionProblem]) -> np.ndarray:
     """hh_correction_t records of the problems, a column at a time (200
     problems: 0.5 ms, record by record 2.2 ms)."""
-    problems = list(problems)
     out = np.zeros(len(problems), dtype=PROBLEM_DTYPE)
     steps: dict = {}            # line-search steps of each (reduction, minimum) seen
     for i, p in enumerate(problems):
         if not device_supported(p, steps):
             raise ValueError(f"problem {i}: the device corrector takes 2x2 problems with at "
                              f"most {_JMAX} line-search steps")
-    if not problems:
+    if len(problems) == 0:
         return out
     for name in ("mu", "tol", "alpha_reduction", "min_alpha", "armijo_c"):
         out[name] = [float(getattr(p, name)) for p in problems]
