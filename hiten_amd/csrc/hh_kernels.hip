@@ -31,6 +31,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <atomic>
 #include <mutex>
 #include <type_traits>
 
@@ -2144,16 +2145,24 @@ StepParams make_sp(double rtol, double atol, double max_step, double min_step,
  * end states 0.64 and 0.62 ms at 8,192, 1.78 and 1.42 ms at 65,536.         */
 constexpr int ROW6_MAX = 4096;
 
-/* End states, one trajectory per lane, of more than SPANS6_MIN trajectories are
- * dealt out by span: 131,072 spans of 0.6 to 3 take 1.24 ms and not 1.92,
- * 262,144 2.2 and not 3.0.  It costs nothing there where all spans are equal
- * (0.90 and 0.89 ms, 1.41 and 1.45 ms).  Fewer trajectories, less than three
- * waves to two SIMDs, keep workgroups of 128: with 256 the CUs are loaded
- * unevenly, and 81,920 equal spans take 0.86 ms and not 0.81 (0.88 with 512).
- * From SPANS6_CU to SPANS6_CU_MAX workgroups of 512 have each its own CU:
- * 114,688 spans of 0.6 to 3 take 1.28 ms with 512, 1.42 with 256, equal ones
- * 0.89 either way (98,304 equal ones 0.88 and 0.85).                        */
-constexpr int SPANS6_MIN = 98304, SPANS6_CU = 114688, SPANS6_CU_MAX = 131072;
+/* Workgroup size for end states, one trajectory per lane, dealt out by span, or
+ * 0 where they are not.  More than 384 trajectories a CU (98,304 on 256 CUs) are:
+ * 131,072 spans of 0.6 to 3 take 1.24 ms and not 1.92, 262,144 2.2 and not 3.0.
+ * It costs nothing there where all spans are equal (0.90 and 0.89 ms, 1.41 and
+ * 1.45 ms).  Fewer trajectories, less than three waves to two SIMDs, keep
+ * workgroups of 128: with 256 the CUs are loaded unevenly, and 81,920 equal spans
+ * take 0.86 ms and not 0.81 (0.88 with 512).  Workgroups of 512 as long as each
+ * has its own CU and at least seven of eight CUs have one: 114,688 spans of 0.6
+ * to 3 take 1.28 ms with 512, 1.42 with 256, equal ones 0.89 either way (98,304
+ * equal ones 0.88 and 0.85).                                                */
+constexpr int spans6_block(long long n, int cus) {
+    return n <= 384LL * cus ? 0 : (n >= 448LL * cus && n <= 512LL * cus ? 512 : 256);
+}
+static_assert(spans6_block(98304, 256) == 0 && spans6_block(98305, 256) == 256 &&
+              spans6_block(114687, 256) == 256 && spans6_block(114688, 256) == 512 &&
+              spans6_block(131072, 256) == 512 && spans6_block(131073, 256) == 256 &&
+              spans6_block(131072, 304) == 256 && spans6_block(155648, 304) == 512,
+              "the sizes measured above, on 256 CUs, and where the lines lie on 304");
 
 template <class M>
 void launch_rk_fixed(int n, int dim, const double* mu, const double* t0p,
@@ -2304,6 +2313,17 @@ int hh_rk8_fixed(int n, int dim, const double* mu, const double* t0, const doubl
                        traj_out, nullptr, variant, block, stream);
 }
 
+/* Compute units of the current device, asked once per device; 0 if that fails */
+static int device_cus() {
+    static std::atomic<int> cus[64];
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+    if ((n = cus[dev].load(std::memory_order_relaxed)) == 0 &&
+        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess)
+        cus[dev].store(n, std::memory_order_relaxed);
+    return n;
+}
+
 /* Resident workgroups of a kernel on the current device (CU count times the
  * occupancy per CU, capped at cap_per_cu when cap_per_cu > 0), queried once
  * per device and kernel: later calls -- e.g. inside a stream capture -- make
@@ -2375,7 +2395,8 @@ int hh_dop853_final_bounded(int wait_polls, int n, int dim, const double* mu, co
     if (dim == 6) {
         if (variant != HH_VARIANT_PLAIN && variant != HH_VARIANT_WIDE)
             return fail(HH_ERR_ARGS, "hh_dop853_final: dim 6 supports the plain and wide variants");
-        const bool by_span = variant != HH_VARIANT_WIDE && block <= 0 && n > SPANS6_MIN;
+        const int cus = variant != HH_VARIANT_WIDE && block <= 0 ? device_cus() : 0;
+        const int by_span = cus > 0 ? spans6_block(n, cus) : 0;
         if (block <= 0) block = 128;
         if (block > 256 || block % 64) return fail(HH_ERR_ARGS, "hh_dop853_final: block must be 64..256, multiple of 64");
         if (variant == HH_VARIANT_WIDE)
@@ -2383,7 +2404,7 @@ int hh_dop853_final_bounded(int wait_polls, int n, int dim, const double* mu, co
                                             nullptr, status, n_acc, n_rej, block, st,
                                             "hh_dop853_final(6, wide) launch");
         if (by_span) {
-            if (n >= SPANS6_CU && n <= SPANS6_CU_MAX)
+            if (by_span == 512)
                 hipLaunchKernelGGL(k_dop853_final6_spans<512>, dim3(blocks_for(n, 512)), dim3(512),
                                    0, st, n, mu, t0, tf, sp, fwd, flip_mask, y0, y_out, status,
                                    n_acc, n_rej);

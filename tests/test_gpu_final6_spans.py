@@ -3,6 +3,7 @@ batch in plain order and against the oracle."""
 
 import numpy as np
 import pytest
+import torch
 
 from hiten_amd import batch, workloads as W
 
@@ -38,3 +39,17 @@ def test_dealing_by_span_changes_no_result(gpu, oracle, n):
             want = oracle.dop853(sys, y[i], np.array([0.0, tf[i]]), rtol=1e-12, atol=1e-12,
                                  max_step=1e4)[0][-1]
             assert np.array_equal(yr[i], want)
+
+
+@pytest.mark.parametrize("per_cu,more", [(384, 0), (384, 1), (448, -1), (448, 0), (512, 0),
+                                         (512, 1)])
+def test_lines_of_the_rule_on_this_device(gpu, per_cu, more):
+    """Either side of every line of the rule, which lie by the device's CUs."""
+    n = per_cu * torch.cuda.get_device_properties(0).multi_processor_count + more
+    rng = np.random.default_rng(n)
+    y = W.planar_seeds(rng, n)
+    tf = rng.uniform(0.01, 0.2, n)
+    a = batch.dop853_final(MU, y, 0.0, tf, variant="plain")
+    b = batch.dop853_final(MU, y, 0.0, tf, variant="plain", block=128)
+    for u, v in zip(vars(a).values(), vars(b).values()):
+        assert torch.equal(u, v)
