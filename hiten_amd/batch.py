@@ -404,6 +404,13 @@ def dop853_final(mu, y0, t0, tf, *, dim: int = 6, rtol: float = 1e-12, atol: flo
                  stream=None) -> FinalResult:
     """Adaptive DOP853 to tf; the state returned is the dense-output value at tf
     (the last row of _propagate_dynsys(..., steps=2)).
+
+    ``variant`` "auto" is the fastest layout for a call that has the GPU to
+    itself (_auto_variant).  Past 4,096 42-d trajectories that is the
+    work-stealing kernel, whose waves stay until the batch ends: a call on
+    another stream may wait for all of it, where "plain" gives its wave slots
+    back workgroup by workgroup.  Its speed, not its results, follows the
+    process-wide settings of hh_set_tuning; the "plain" kernel reads none.
     """
     # a graph recorded on the launch stream alone keeps neither a workspace nor
     # a hand-out order of this call's alive
