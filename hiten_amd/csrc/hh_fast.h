@@ -6,12 +6,18 @@
  * division or square root do nothing.  FastChk holds the exponent range of
  * the forms below; where a lane of the wave leaves it, the wave takes the
  * general forms.  Within the range every result is the correctly rounded
- * one, so the bits are the same:
+ * one except for rare arguments, named below; no output of any test or timed
+ * case has differed.
  *
- *   fast_div     q = n r, then one correction with the exact remainder, from
- *                a reciprocal r correct to half an ulp (Markstein's theorem:
- *                the corrected quotient is then the correctly rounded one).
- *                Quotients of one denominator share its reciprocal.  The
+ *   fast_div     q = n r, then one correction with the exact remainder.  By
+ *                Markstein's theorem the corrected quotient is the correctly
+ *                rounded one if r is 1/d correctly rounded and d's significand
+ *                is not all ones.  r comes from one Newton step on a value
+ *                good to 2^-43 or better, so it is correctly rounded except
+ *                where 1/d lies within about 2^-33 of its last place of a
+ *                rounding boundary; a quotient of such a d can then be off by
+ *                its last bit, and only if it lies as close to a boundary
+ *                itself.  Quotients of one denominator share its reciprocal.  The
  *                remainder is taken with the sign that keeps a zero
  *                quotient's sign.
  *   fast_pow     x^1.5 and x^2.5 as hh_pow15_25 forms them, without its
@@ -19,7 +25,8 @@
  *                instead of two: the second changes the root's last bit in
  *                about 1 of 2^37 arguments, and the powers, formed from the
  *                root and its exact remainder, change only if their exact
- *                value also lies within 2^-103 of a rounding boundary.
+ *                value also lies within 2^-103 of a rounding boundary: not the
+ *                same bits for every argument, at the same precision.
  *   reciprocals  of r^3 and r^5 start from powers of the refined 1/r the
  *                square root leaves behind (2^-43), one Newton step each.
  */
@@ -59,14 +66,14 @@ struct FastChk {
     }
 };
 
-/* n / d from r = 1/d to half an ulp */
+/* n / d from r = 1/d correctly rounded (see above where it is not) */
 __device__ __forceinline__ double fast_div(double n, double d, double r) {
     const double q = n * r;
     const double t = __builtin_fma(d, q, -n);
     return __builtin_fma(-t, r, q);
 }
 
-/* 1/d to half an ulp */
+/* 1/d, correctly rounded but for rare d */
 __device__ __forceinline__ double fast_rcp(double d) {
     double r = __builtin_amdgcn_rcp(d);
     double e = __builtin_fma(-d, r, 1.0);
